@@ -18,10 +18,11 @@
 // runs:
 //   filter x,y,z (in place)           filterq      src/comsolver.F90:514
 //   qswap i, j, k parts                qswap        src/parallel.F90:4849
-//   gradient sweeps x,y,z              gradcal      src/comsolver.F90:244
-//   k_gflux (pointwise)                sigma, qflux and the axis fluxes
-//                                      G = Fv - F of convrsdcal6/diffrsdcal6
-//   flux sweeps x,y,z                  one derivative of G per axis into qrhs
+//   gradient sweeps y,z                gradcal      src/comsolver.F90:244
+//   k_row_flux (x rows)                the x gradient, sigma, qflux, the axis
+//                                      fluxes G = Fv - F of convrsdcal6/
+//                                      diffrsdcal6 and the x derivative of G
+//   flux sweeps y,z                    one derivative of G per axis into qrhs
 //                                      (qrhs=-qrhs folded in); the z sweep
 //                                      applies the RK3 combine
 //   k_prim                             updatefvar   src/mainloop.F90:476
@@ -921,8 +922,17 @@ __device__ __forceinline__ void q2fvar(const PtArgs& a, const double qv[5], long
 }
 #pragma clang fp contract(fast)
 
+// the constants of the viscous terms
+struct ViscConst {
+    double reynolds, prandtl, const5, tempconst, tempconst1;
+};
+__device__ __forceinline__ ViscConst visc_const(const PtArgs& a)
+{
+    return {a.reynolds, a.prandtl, a.const5, a.tempconst, a.tempconst1};
+}
+
 // miucal, src/fludyna.F90:791-820
-__device__ __forceinline__ double miucal(const PtArgs& a, double t)
+__device__ __forceinline__ double miucal(const ViscConst& a, double t)
 {
     return t * sqrt(t) * a.tempconst1 / (t + a.tempconst);
 }
@@ -1109,22 +1119,32 @@ __host__ __device__ __forceinline__ void dd_add(double& ah, double& al, double b
 // The per-node terms of kenergycal / enstophycal / diss_rate_cal
 // (src/statistic.F90:870-1042): rho |u|^2, rho |omega|^2 and
 // 2 mu (S:S - (div u)^2 / 3)
-__device__ __forceinline__ void stats_terms(const PtArgs& a, long gi, double& ke, double& en,
-                                            double& di)
+__device__ __forceinline__ void stats_of(const ViscConst& a, double rho, const double* uvw, double T,
+                                         const double* dv, double& ke, double& en, double& di)
 {
-    const double rho = a.prim[0][gi];
-    const double u = a.prim[1][gi], v = a.prim[2][gi], w = a.prim[3][gi];
+    const double u = uvw[0], v = uvw[1], w = uvw[2];
     ke = rho * (u * u + v * v + w * w);
-    const double d11 = a.dvel[0][gi], d12 = a.dvel[1][gi], d13 = a.dvel[2][gi];
-    const double d21 = a.dvel[3][gi], d22 = a.dvel[4][gi], d23 = a.dvel[5][gi];
-    const double d31 = a.dvel[6][gi], d32 = a.dvel[7][gi], d33 = a.dvel[8][gi];
+    const double d11 = dv[0], d12 = dv[1], d13 = dv[2];
+    const double d21 = dv[3], d22 = dv[4], d23 = dv[5];
+    const double d31 = dv[6], d32 = dv[7], d33 = dv[8];
     const double o1 = d32 - d23, o2 = d13 - d31, o3 = d21 - d12;
     en = rho * (o1 * o1 + o2 * o2 + o3 * o3);
-    const double miu = miucal(a, a.prim[5][gi]) / a.reynolds;
+    const double miu = miucal(a, T) / a.reynolds;
     const double s12 = 0.5 * (d12 + d21), s13 = 0.5 * (d13 + d31), s23 = 0.5 * (d23 + d32);
     const double div = d11 + d22 + d33;
     di = 2.0 * miu * (d11 * d11 + d22 * d22 + d33 * d33 +
                       2.0 * (s12 * s12 + s13 * s13 + s23 * s23) - (1.0 / 3.0) * (div * div));
+}
+
+// stats_of at a node of the stored primitives and gradients
+__device__ __forceinline__ void stats_terms(const PtArgs& a, long gi, double& ke, double& en,
+                                            double& di)
+{
+    const double uvw[3] = {a.prim[1][gi], a.prim[2][gi], a.prim[3][gi]};
+    double dv[9];
+#pragma unroll
+    for (int c = 0; c < 9; ++c) dv[c] = a.dvel[c][gi];
+    stats_of(visc_const(a), a.prim[0][gi], uvw, a.prim[5][gi], dv, ke, en, di);
 }
 
 // The block's sums of (ke, en, di) into part[6 * blockIdx.x ...] as
@@ -1179,16 +1199,14 @@ __device__ __forceinline__ NodeIn load_node(const PtArgs& a, long gi)
 
 // sigma and qflux of diffrsdcal6 (src/solver.F90:2434-2546, turbmode none)
 // at one node from its gradients, temperature and velocity:
-// sg = (s11, s12, s13, s22, s23, s33), qf(1:3)
-__device__ __forceinline__ void sigma_of(const PtArgs& a, long gi, const double* uvw, double* sg,
-                                         double* qf)
+// sg = (s11, s12, s13, s22, s23, s33), qf(1:3).  Here and in gflux_of the
+// fused multiply-adds are written out and the compiler adds none, so that
+// every kernel that evaluates a node's fluxes rounds them alike.
+#pragma clang fp contract(off)
+__device__ __forceinline__ void sigma_from(const ViscConst& a, const double* dv, const double* dt,
+                                           double T, const double* uvw, double* sg, double* qf)
 {
-    double dv[9], dt[3];
-#pragma unroll
-    for (int c = 0; c < 9; ++c) dv[c] = a.dvel[c][gi];
-#pragma unroll
-    for (int c = 0; c < 3; ++c) dt[c] = a.dtmp[c][gi];
-    const double miu = miucal(a, a.prim[5][gi]) / a.reynolds;
+    const double miu = miucal(a, T) / a.reynolds;
     const double d11 = dv[0], d12 = dv[1], d13 = dv[2];
     const double d21 = dv[3], d22 = dv[4], d23 = dv[5];
     const double d31 = dv[6], d32 = dv[7], d33 = dv[8];
@@ -1201,9 +1219,22 @@ __device__ __forceinline__ void sigma_of(const PtArgs& a, long gi, const double*
     const double g4 = miu2 * (s22 - skk), g5 = miu2 * s23, g6 = miu2 * (s33 - skk);
     sg[0] = g1; sg[1] = g2; sg[2] = g3; sg[3] = g4; sg[4] = g5; sg[5] = g6;
     const double u = uvw[0], v = uvw[1], w = uvw[2];
-    qf[0] = hcc * dt[0] + g1 * u + g2 * v + g3 * w;
-    qf[1] = hcc * dt[1] + g2 * u + g4 * v + g5 * w;
-    qf[2] = hcc * dt[2] + g3 * u + g5 * v + g6 * w;
+    qf[0] = fma(g3, w, fma(g2, v, fma(g1, u, hcc * dt[0])));
+    qf[1] = fma(g5, w, fma(g4, v, fma(g2, u, hcc * dt[1])));
+    qf[2] = fma(g6, w, fma(g5, v, fma(g3, u, hcc * dt[2])));
+}
+#pragma clang fp contract(fast)
+
+// the same from the stored gradients and temperature
+__device__ __forceinline__ void sigma_of(const PtArgs& a, long gi, const double* uvw, double* sg,
+                                         double* qf)
+{
+    double dv[9], dt[3];
+#pragma unroll
+    for (int c = 0; c < 9; ++c) dv[c] = a.dvel[c][gi];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) dt[c] = a.dtmp[c][gi];
+    sigma_from(visc_const(a), dv, dt, a.prim[5][gi], uvw, sg, qf);
 }
 
 // The flux of axis d that the flux sweep differentiates, G = Fv - F, at one
@@ -1214,6 +1245,7 @@ __device__ __forceinline__ void sigma_of(const PtArgs& a, long gi, const double*
 // The derivative is linear, so the reference's two passes (qrhs = -sum D F,
 // then qrhs += sum D Fv) become one derivative of Fv - F per axis; only the
 // summation order differs.
+#pragma clang fp contract(off)
 __device__ __forceinline__ void gflux_of(const PtArgs& a, int d, double xn, const NodeIn& n,
                                          const double* sg, const double* qf, double* out)
 {
@@ -1229,7 +1261,7 @@ __device__ __forceinline__ void gflux_of(const PtArgs& a, int d, double xn, cons
             const double qm = n.q[m];
             double fc;
             if (m == 4) fc = (qm + p) * uu;
-            else if (m == d + 1) fc = qm * uu + p;
+            else if (m == d + 1) fc = fma(qm, uu, p);
             else fc = qm * uu;
             if (m == 0 || !a.visc) out[m] = -fc;
             else out[m] = (m < 4 ? sg[sidx[d][m - 1]] : qf[d]) - fc;
@@ -1244,16 +1276,17 @@ __device__ __forceinline__ void gflux_of(const PtArgs& a, int d, double xn, cons
         double fi;
         if (m == 0) fi = jc * qm * uu;
         else if (m == 4) fi = jc * (qm + p) * uu;
-        else if (m == d + 1) fi = jc * (qm * uu + xn * p);
+        else if (m == d + 1) fi = jc * fma(qm, uu, xn * p);
         else fi = jc * (qm * uu);
         if (m == 0 || !a.visc) {
             out[m] = -fi;
         } else {
             const double sv = m < 4 ? sg[sidx[d][m - 1]] : qf[d];
-            out[m] = (sv * xn) * jc - fi;
+            out[m] = fma(sv * xn, jc, -fi);
         }
     }
 }
+#pragma clang fp contract(fast)
 
 // gflux_of with the three metric components of axis d at the node (a grid
 // with general metrics): U = dxi(d,:).u, the pressure on every momentum
@@ -1511,6 +1544,264 @@ __device__ __forceinline__ void prim_body(const PtArgs& a, unsigned bid)
 }
 
 __global__ __launch_bounds__(256) void k_prim(PtArgs a) { prim_body(a, blockIdx.x); }
+
+// -------------------------------------------------------------- row kernel
+//
+// An x line is a row of memory, so one wavefront can hold a row of several
+// quantities at once: the x sweeps then fuse with the pointwise work on
+// either side of them, which the y/z tiles (one quantity per workgroup) do
+// not allow.  A workgroup is one wavefront and one interior row (j, k); the
+// quantities' lines sit in LDS rows (node n at ln[n + HM]), each
+// half-wavefront solves one quantity with solve_line, and the wavefront
+// takes the row's nodes 64 at a time for everything else.
+
+struct RowArgs {
+    PtArgs p;
+    LineTab tab;      // the x line system of the derivative
+    int rs;           // LDS row stride
+    double* gx[4];    // dvel(1:3,1), dtmp(1), written when keep_grad
+    int keep_grad;
+    double* qrhs[5];
+};
+
+// doubles per x halo node of k_row_flux's side rows: the image's sigma (3) and
+// heat flux, the node's q (5), p, u and J
+constexpr int ROW_STRIP = 12;
+
+__device__ __forceinline__ void wave_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// the solved rows of a line go back to their nodes' slots; the padding rows
+// past R would run into the next line
+template <int L>
+__device__ __forceinline__ void row_back(const LineTab& tab, int sub, double* ln,
+                                         const double (&x)[L])
+{
+    double* o = ln + HM + tab.first + sub * L;
+#pragma unroll
+    for (int t = 0; t < L; ++t)
+        if (sub * L + t < tab.R) o[t] = x[t];
+}
+
+// The x gradient, sigma, the heat flux, the fluxes G of the three axes and
+// the x flux derivative of one row, in the order and operations of the x
+// gradient sweep, k_gflux and the x flux sweep (whose results it equals bit
+// for bit), for viscous flow on rectilinear metrics: u, v, w, T of the row
+// are staged and differentiated in LDS, the y and z gradients (already
+// stored by their sweeps) complete the node's sigma, G_y and G_z go to
+// memory, G_x stays in LDS, where it is differentiated, and qrhs takes the
+// result.  The x halo strips take sigma and the heat flux of their periodic
+// images, which are nodes of the same row (side rows in LDS); the y and z
+// halo rows of which this row is the image are written here as in k_gflux.
+// Memory bound: 18 doubles in and 15 out per node, where the three kernels
+// moved 55 (the x gradients, G_x and the fluxes' second reading of u, v, w, T
+// stay on the chip).  Per stage, three kernels -> one: 256^3 1689 -> 1060 us
+// (4.25 TB/s), 128^3 259 -> 152 us, 64^3 56 -> 33 us.  Registers: up to L = 6
+// the table of the line system is held over the solves within 128 of them (4
+// waves per SIMD); above, the five LDS rows allow 3 waves.
+template <int L, bool STATS>
+__global__ __launch_bounds__(64, L <= 6 ? 4 : 3) void k_row_flux(RowArgs ra)
+{
+    extern __shared__ double buf[];
+    const PtArgs& a = ra.p;
+    const int n = a.g.n[0];
+    const int lend = line_end_i(n);
+    const unsigned nj = (unsigned)a.g.n[1] + 1;
+    const unsigned kk = blockIdx.x / nj;
+    const int j = (int)(blockIdx.x - kk * nj), k = (int)kk;
+    const int lane = threadIdx.x, half = lane >> 5, sub = lane & 31;
+    const unsigned g0 = (unsigned)gidx(a.g, 0, j, k) * 8u;  // byte offset of node 0
+    const int rs = ra.rs;
+    double* const side = buf + 5 * rs;
+    // lanes 0-9: the halo nodes -5..-1, n+1..n+5
+    const int hc = lane < HM ? lane - HM : n + 1 + lane - HM;
+
+    // the inputs of G at byte offset b (32-bit offsets throughout: 64-bit
+    // addresses of the 25 fields would be kept in registers over the loop)
+    auto load = [&](unsigned b, NodeIn& v) {
+#pragma unroll
+        for (int m = 0; m < 3; ++m) v.u[m] = ldc(a.prim[1 + m], b);
+#pragma unroll
+        for (int m = 0; m < 5; ++m) v.q[m] = ldc(a.q[m], b);
+        v.p = ldc(a.prim[4], b);
+        v.jc = a.juni ? a.j0 : ldc(a.jac, b);
+    };
+
+    // ---------------- stage u, v, w, T
+    constexpr int E = (32 * L + 4 + 63) / 64;  // n + 1 + 2 HM <= 32 L + 4 nodes
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+        const int c = lane + 64 * e - HM;
+        if (c <= n + HM) {
+#pragma unroll
+            for (int m = 0; m < 4; ++m)
+                buf[m * rs + TG + HM + c] = ldc(a.prim[m < 3 ? 1 + m : 5], g0 + (unsigned)(c * 8));
+        }
+    }
+    if (a.per[0] && lane < 2 * HM) {
+        NodeIn nh;
+        load(g0 + (unsigned)(hc * 8), nh);
+        double* o = side + ROW_STRIP * lane + 4;
+#pragma unroll
+        for (int m = 0; m < 5; ++m) o[m] = nh.q[m];
+        o[5] = nh.p;
+        o[6] = nh.u[0];
+        o[7] = nh.jc;
+    }
+    wave_sync();
+
+    // ---------------- gradcal along x
+#pragma unroll 1
+    for (int pr = 0; pr < 2; ++pr) {
+        double* ln = buf + (2 * pr + half) * rs + TG;
+        double x[L];
+        solve_line<L, OP_DERIV>(ln, ra.tab, nullptr, x);
+        const int rb = ra.tab.first + sub * L;
+#pragma unroll
+        for (int t = 0; t < L; ++t) x[t] *= a.xi[0][min(max(rb + t, -HM), n + HM) + HM];
+        row_back<L>(ra.tab, sub, ln, x);
+    }
+    wave_sync();
+
+    // ---------------- sigma, heat flux, G
+    const int hj = a.per[1] ? halo_of_image(j, a.g.n[1]) : NO_HALO;
+    const int hk = a.per[2] ? halo_of_image(k, a.g.n[2]) : NO_HALO;
+    const unsigned dhj = (unsigned)((hj - j) * (int)a.g.s[1]) * 8u;
+    const unsigned dhk = (unsigned)((hk - k) * (int)a.g.s[2]) * 8u;
+    const double xy = a.xi[1][j + HM], xz = a.xi[2][k + HM];
+    double st[3] = {0.0, 0.0, 0.0};
+#pragma unroll 1
+    for (int c0 = 0; c0 < lend; c0 += 64) {
+        const int c = c0 + lane;
+        const unsigned b = g0 + (unsigned)(c * 8);
+        if (c <= n) {
+            NodeIn nd;
+            double dv[9], dt[3];
+#pragma unroll
+            for (int m = 0; m < 3; ++m) {
+                dv[3 * m + 1] = ldb(a.dvel[3 * m + 1], b);
+                dv[3 * m + 2] = ldb(a.dvel[3 * m + 2], b);
+            }
+            dt[1] = ldb(a.dtmp[1], b);
+            dt[2] = ldb(a.dtmp[2], b);
+            const double T = ldc(a.prim[5], b);
+            load(b, nd);
+            const double rho = STATS ? ldc(a.prim[0], b) : 0.0;
+            double sg[6], qf[3];
+            // (opaque: the reciprocals of the constants would otherwise be
+            // held in registers over the loop)
+            ViscConst vc = visc_const(a);
+            asm volatile("" : "+s"(vc.reynolds), "+s"(vc.prandtl), "+s"(vc.const5));
+            double* const ln = buf + TG + HM + c;
+#pragma unroll
+            for (int m = 0; m < 3; ++m) dv[3 * m] = ln[m * rs];
+            dt[0] = ln[3 * rs];
+            sigma_from(vc, dv, dt, T, nd.u, sg, qf);
+            if (STATS && c >= 1 && j >= 1 && k >= 1) {
+                double t[3];
+                stats_of(vc, rho, nd.u, T, dv, t[0], t[1], t[2]);
+#pragma unroll
+                for (int m = 0; m < 3; ++m) st[m] += t[m];
+            }
+            if (ra.keep_grad) {
+#pragma unroll
+                for (int m = 0; m < 4; ++m) stb(ra.gx[m], b, m < 3 ? dv[3 * m] : dt[0]);
+            }
+            double out[5];
+            gflux_of(a, 0, a.xi[0][c + HM], nd, sg, qf, out);
+#pragma unroll
+            for (int m = 0; m < 5; ++m) ln[m * rs] = out[m];
+            const int ih = halo_of_image(c, n);
+            if (ih != NO_HALO) {
+                double* sv = side + ROW_STRIP * (ih < 0 ? ih + HM : ih - n - 1 + HM);
+                sv[0] = sg[0];
+                sv[1] = sg[1];
+                sv[2] = sg[2];
+                sv[3] = qf[0];
+            }
+            gflux_of(a, 1, xy, nd, sg, qf, out);
+#pragma unroll
+            for (int m = 0; m < 5; ++m) stb(a.gfl[5 + m], b, out[m]);
+            gflux_of(a, 2, xz, nd, sg, qf, out);
+#pragma unroll
+            for (int m = 0; m < 5; ++m) stb(a.gfl[10 + m], b, out[m]);
+            if (hj != NO_HALO) {
+                const unsigned h = b + dhj;
+                load(h, nd);
+                gflux_of(a, 1, a.xi[1][hj + HM], nd, sg, qf, out);
+#pragma unroll
+                for (int m = 0; m < 5; ++m) stb(a.gfl[5 + m], h, out[m]);
+            }
+            if (hk != NO_HALO) {
+                const unsigned h = b + dhk;
+                load(h, nd);
+                gflux_of(a, 2, a.xi[2][hk + HM], nd, sg, qf, out);
+#pragma unroll
+                for (int m = 0; m < 5; ++m) stb(a.gfl[10 + m], h, out[m]);
+            }
+        } else if (c < lend) {
+            // the rest of the line of node n, which nothing reads
+#pragma unroll
+            for (int m = 0; m < 10; ++m) stb(a.gfl[5 + m], b, 0.0);
+#pragma unroll
+            for (int m = 0; m < 5; ++m) {
+                if (hj != NO_HALO) stb(a.gfl[5 + m], b + dhj, 0.0);
+                if (hk != NO_HALO) stb(a.gfl[10 + m], b + dhk, 0.0);
+            }
+            if (ra.keep_grad) {
+#pragma unroll
+                for (int m = 0; m < 4; ++m) stb(ra.gx[m], b, 0.0);
+            }
+        }
+    }
+    wave_sync();
+    if (a.per[0] && lane < 2 * HM) {
+        const double* sv = side + ROW_STRIP * lane;
+        const double sg[6] = {sv[0], sv[1], sv[2], 0, 0, 0}, qf[3] = {sv[3], 0, 0};
+        double out[5];
+        NodeIn nh;
+#pragma unroll
+        for (int m = 0; m < 5; ++m) nh.q[m] = sv[4 + m];
+        nh.p = sv[9];
+        nh.u[0] = sv[10];
+        nh.jc = sv[11];
+        gflux_of(a, 0, a.xi[0][hc + HM], nh, sg, qf, out);
+#pragma unroll
+        for (int m = 0; m < 5; ++m) buf[m * rs + TG + HM + hc] = out[m];
+    }
+    wave_sync();
+
+    // ---------------- the x flux derivative
+#pragma unroll 1
+    for (int pr = 0; pr < 3; ++pr) {
+        // (the last pass: both halves solve quantity 4 and store alike)
+        double* ln = buf + min(2 * pr + half, 4) * rs + TG;
+        double x[L];
+        solve_line<L, OP_DERIV>(ln, ra.tab, nullptr, x);
+        row_back<L>(ra.tab, sub, ln, x);
+    }
+    wave_sync();
+    // (past node n: the dead rest of its line, any value)
+    for (int c = lane; c < lend; c += 64) {
+#pragma unroll
+        for (int m = 0; m < 5; ++m)
+            stb(ra.qrhs[m], g0 + (unsigned)(c * 8), buf[m * rs + TG + HM + min(c, n)]);
+    }
+    if (STATS) {
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1)
+#pragma unroll
+            for (int m = 0; m < 3; ++m) st[m] += __shfl_xor(st[m], off, 64);
+        if (lane == 0)
+            for (int m = 0; m < 3; ++m) {
+                a.part[6 * (long)blockIdx.x + 2 * m] = st[m];
+                a.part[6 * (long)blockIdx.x + 2 * m + 1] = 0.0;
+            }
+    }
+}
 
 // gradcal's metric combination on a grid with general metrics
 // (src/comsolver.F90:304-318, 344-358, 384-398): the sweeps left the
@@ -3699,6 +3990,39 @@ int launch_sweep(astr_ctx* c, const SweepArgs& a, hipStream_t st = nullptr)
     return fail(ASTR_E_ARG, "unknown pass");
 }
 
+// ---- row kernel (x lines of all quantities of a row)
+
+RowArgs row_args(astr_ctx* c)
+{
+    RowArgs r{};
+    r.p = pt_args(c);
+    r.tab = c->tab[0][OP_DERIV];
+    r.rs = (TG + c->g.n[0] + 1 + 2 * HM) | 1;
+    for (int m = 0; m < 3; ++m) r.gx[m] = c->dvel[3 * m];
+    r.gx[3] = c->dtmp[0];
+    for (int m = 0; m < 5; ++m) r.qrhs[m] = c->qrhs[m];
+    return r;
+}
+
+template <bool STATS>
+int launch_row_flux(astr_ctx* c, const RowArgs& r)
+{
+    const dim3 grid((unsigned)((c->g.n[1] + 1) * (c->g.n[2] + 1)));
+    const size_t lds = sizeof(double) * (5 * (size_t)r.rs + ROW_STRIP * 2 * HM);
+    switch (c->L[0]) {
+#define CASE(LL)                                                                          \
+    case LL:                                                                              \
+        hipLaunchKernelGGL((k_row_flux<LL, STATS>), grid, dim3(64), lds, c->stream, r);   \
+        break;
+        CASE(1) CASE(2) CASE(3) CASE(4) CASE(5) CASE(6) CASE(7) CASE(8)
+        CASE(9) CASE(10) CASE(11) CASE(12) CASE(13) CASE(14) CASE(15) CASE(16)
+#undef CASE
+    default:
+        return fail(ASTR_E_UNSUPPORTED, "line too long");
+    }
+    HIPCHK(hipGetLastError());
+    return ASTR_OK;
+}
 
 // ---- transposed sweeps
 
@@ -3939,10 +4263,18 @@ int do_boucon(astr_ctx* c)
 // primitives.
 const double RKC[3][3] = {{1.0, 0.0, 1.0}, {0.75, 0.25, 0.25}, {1.0 / 3.0, 2.0 / 3.0, 2.0 / 3.0}};
 
+// viscous flow on rectilinear metrics: the x part of the gradient and of
+// the flux derivative runs with the fluxes in k_row_flux
+bool row_flux_ok(const astr_ctx* c)
+{
+    return !c->curv && c->p.diffterm != 0 && c->p.variant == 0;
+}
+
 int do_flux_sweeps(astr_ctx* c, int rk_stage, double dt, double* const* qo = nullptr,
                    bool qsraw = false)
 {
-    for (int d = 0; d < 3; ++d) {
+    // the x derivative comes with the fluxes where the row kernel runs
+    for (int d = row_flux_ok(c) ? 1 : 0; d < 3; ++d) {
         SweepArgs a = sweep_args(c, d, PASS_RHS);
         if (qo)
             for (int m = 0; m < 5; ++m) a.qo[m] = qo[m];
@@ -3987,6 +4319,31 @@ int do_gflux(astr_ctx* c, double* stats_slot = nullptr)
     }
     HIPCHK(hipGetLastError());
     return ASTR_OK;
+}
+
+// gradcal, sigma/qflux and G, and the x flux derivative into qrhs.  Where
+// k_row_flux runs it takes the x part with the pointwise work; keep_grad: it
+// also stores the x gradients (what the statistics, the reversal and
+// astr_download_rhs read).  General metrics combine the three axes'
+// derivatives before the fluxes, so they keep the separate launches, as do
+// the mini-app's forms and inviscid flow.  mark: the timing slot between the
+// gradient and the fluxes.
+int do_grad(astr_ctx* c);
+int time_mark(astr_ctx* c, int slot);
+int do_central_flux(astr_ctx* c, bool keep_grad, double* stats_slot = nullptr, int mark = -1)
+{
+    if (!row_flux_ok(c)) {
+        TRY(do_grad(c));
+        if (mark >= 0) TRY(time_mark(c, mark));
+        return do_gflux(c, stats_slot);
+    }
+    for (int d = 1; d < 3; ++d) TRY(launch_sweep(c, sweep_args(c, d, PASS_GRAD)));
+    if (mark >= 0) TRY(time_mark(c, mark));
+    RowArgs r = row_args(c);
+    r.keep_grad = keep_grad;
+    if (!stats_slot) return launch_row_flux<false>(c, r);
+    TRY(launch_row_flux<true>(c, r));
+    return stats_finish(c, (long)(c->g.n[1] + 1) * (c->g.n[2] + 1), stats_slot);
 }
 
 int ndims_of(const astr_ctx* c) { return c->g.n[2] == 0 ? 2 : 3; }
@@ -4184,8 +4541,6 @@ int do_grad(astr_ctx* c)
     return ASTR_OK;
 }
 
-int time_mark(astr_ctx* c, int slot);
-
 int do_rhscal(astr_ctx* c, bool timed = false)
 {
     if (c->p.convection != 0) {
@@ -4210,8 +4565,7 @@ int do_rhscal(astr_ctx* c, bool timed = false)
         }
         return ASTR_OK;
     }
-    TRY(do_grad(c));
-    TRY(do_gflux(c));
+    TRY(do_central_flux(c, true));
     return do_flux_sweeps(c, 0, 0.0);
 }
 
@@ -4312,7 +4666,10 @@ int time_mark(astr_ctx* c, int slot)
 // step, so no qsave = q J is stored (5 fields per step fewer).  The
 // buffers then alternate from step to step; a generation bump makes a
 // batch that holds this context rebuild its launches.
-int do_step(astr_ctx* c, double dt, double* stats_slot, bool timed, bool alt = false)
+// last: no other step follows at once, so the x gradients of the last stage
+// are kept for the calls that read them (statistics, astr_download_rhs).
+int do_step(astr_ctx* c, double dt, double* stats_slot, bool timed, bool alt = false,
+            bool last = true)
 {
     c->bc_dt = dt;  // boucon's outflow reads the step's deltat
     // timing families: 0 filter, 1 boucon and qswap, 2 grad, 3 central:
@@ -4338,10 +4695,8 @@ int do_step(astr_ctx* c, double dt, double* stats_slot, bool timed, bool alt = f
                 TRY(launch_pt(c, k_bchomo, 2L * HM * (nj * nk + ni * nk + ni * nj), pt_args(c)));
             }
             if (timed) TRY(time_mark(c, 2));
-            TRY(do_grad(c));
-            if (timed) TRY(time_mark(c, 3));
-            // rkfirst's statistics of the stage-1 state, summed by k_gflux
-            TRY(do_gflux(c, s == 1 ? stats_slot : nullptr));
+            // rkfirst's statistics of the stage-1 state, summed with the fluxes
+            TRY(do_central_flux(c, s == 3, s == 1 ? stats_slot : nullptr, timed ? 3 : -1));
             if (timed) TRY(time_mark(c, 4));
             if (timed) TRY(time_mark(c, 5));
             TRY(do_flux_sweeps(c, s, dt));
@@ -4371,12 +4726,16 @@ int do_step(astr_ctx* c, double dt, double* stats_slot, bool timed, bool alt = f
         TRY(do_boucon(c));
         TRY(do_qswap(c));
         if (timed) TRY(time_mark(c, 2));
-        TRY(do_grad(c));
-        if (timed) TRY(time_mark(c, 3));
         // rkfirst's statcal sees the stage-1 state and its gradients; the
-        // central path sums it inside k_gflux, which loads the same inputs
-        if (!upwind) TRY(do_gflux(c, s == 1 ? stats_slot : nullptr));
-        else if (sensor_on(c)) TRY(do_sensor(c));
+        // central path sums it with the fluxes, which load the same inputs
+        if (!upwind) {
+            TRY(do_central_flux(c, s == 3 && last, s == 1 ? stats_slot : nullptr,
+                                timed ? 3 : -1));
+        } else {
+            TRY(do_grad(c));
+            if (timed) TRY(time_mark(c, 3));
+            if (sensor_on(c)) TRY(do_sensor(c));
+        }
         if (timed) TRY(time_mark(c, 4));
         if (upwind && s == 1 && stats_slot) TRY(launch_stats(c, stats_slot));
         if (timed) TRY(time_mark(c, 5));
@@ -4588,8 +4947,7 @@ int segment_fwd(astr_ctx* c, long nstates, long nst, double dt)
             for (int m = 0; m < 9; ++m) c->dvel[m] = st.dvel[m];
             for (int m = 0; m < 3; ++m) c->dtmp[m] = st.dtmp[m];
             TRY(do_qswap(c));
-            TRY(do_grad(c));
-            TRY(do_gflux(c));
+            TRY(do_central_flux(c, true));
             TRY(do_flux_sweeps(c, s, dt, st.qn));
             for (int m = 0; m < 5; ++m) c->q[m] = st.qn[m];
             if (k + 1 < nst) {
@@ -5296,7 +5654,9 @@ int astr_create(const astr_params* p, int32_t device, astr_ctx** out)
     // partial sums of k_stats (one workgroup per 256 nodes) or of k_gflux's
     // statistics (one per workgroup)
     c->npart = ((long)dims[0] * dims[1] * std::max(dims[2], 1) + 255) / 256;
-    if (dims[2] > 0) c->npart = std::max(c->npart, gflux_blocks(c->g));
+    if (dims[2] > 0)
+        c->npart = std::max(std::max(c->npart, gflux_blocks(c->g)),
+                            (long)(dims[1] + 1) * (dims[2] + 1));
     c->host_part.resize(6 * c->npart);
     // the partials, then the second-level partials of the statistics
     if (hipMalloc(&c->part, sizeof(double) * 6 * (c->npart + STATS_FIN)) != hipSuccess)
@@ -5663,7 +6023,8 @@ static int rk3_steps(astr_ctx* c, int32_t nsteps, double dt, double* stats, bool
     int done = 0;
     for (int s = 0; s < nsteps; ++s) {
         const int slot = s - done;
-        TRY(do_step(c, dt, stats ? c->stats_dev + 3 * slot : nullptr, c->timing == 1, true));
+        TRY(do_step(c, dt, stats ? c->stats_dev + 3 * slot : nullptr, c->timing == 1, true,
+                    s + 1 == nsteps));
         if (stats && (slot + 1 == STATS_SLOTS || s + 1 == nsteps)) {
             HIPCHK(hipMemcpyAsync(stats + 3 * (long)done, c->stats_dev,
                                   sizeof(double) * 3 * (slot + 1), hipMemcpyDeviceToHost,
@@ -6305,7 +6666,7 @@ int astr_adjoint_record(astr_ctx* c, int32_t nsteps, double dt, int32_t ckpt, do
         if (seg == nseg - 1) {
             TRY(segment_fwd(c, nstates, 3 * (t1 - t0), dt));
         } else {
-            for (long t = t0; t < t1; ++t) TRY(do_step(c, dt, nullptr, false, true));
+            for (long t = t0; t < t1; ++t) TRY(do_step(c, dt, nullptr, false, true, false));
         }
     }
     TRY(save_state(c, nseg));
