@@ -1098,6 +1098,30 @@ __global__ void k_qswap2d_plane(PtArgs a)
     a.prim[4][gi + a.g.s[2]] = p;
 }
 
+// The same within a step: k_rk has just written the primitives of every
+// node from its q, so only the nodes that boucon set since, those of the
+// edges i = 0, n and j = 0, n, are refreshed.
+__global__ void k_qswap2d_edge(PtArgs a)
+{
+    const int ni = a.g.n[0] + 1, nj = a.g.n[1] + 1;
+    int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= 2 * (ni + nj)) return;
+    int i, j;
+    if (t < 2 * ni) {
+        i = t % ni;
+        j = t < ni ? 0 : nj - 1;
+    } else {
+        t -= 2 * ni;
+        j = t % nj;
+        i = t < nj ? 0 : ni - 1;
+        if (j == 0 || j == nj - 1) return;  // the corners are the rows' own
+    }
+    const long gi = gidx(a.g, i, j, 0);
+    double qv[5];
+    for (int m = 0; m < 5; ++m) qv[m] = a.q[m][gi];
+    q2fvar(a, qv, gi);
+}
+
 // s + e = a + b exactly (Knuth's TwoSum; plain IEEE additions)
 __host__ __device__ __forceinline__ void two_sum(double a, double b, double& s, double& e)
 {
@@ -1503,7 +1527,7 @@ __global__ void k_rk(PtArgs a)
     int i, j, k;
     interior_ijk(a.g, p, i, j, k);
     const long gi = gidx(a.g, i, j, k);
-    const double jc = a.jac[gi];
+    const double jc = a.juni ? a.j0 : a.jac[gi];
     // every operand is read before the first store (which could alias it)
     double qo[5], qs[5], qr[5], qv[5];
 #pragma unroll
@@ -2448,7 +2472,9 @@ struct UwdArgs {
     int iss, iee;        // nodes the split fluxes are taken on
     int a0, a1, b0, b1;  // line ranges over the two other axes
     int ntile_line, ntile_a;
-    int recon, lchar, sensor, last;
+    int recon, lchar, sensor, first, last;
+    int juni;               // jac is j0 everywhere
+    double j0;
     double bfac, gamma, mach;
     const double* q[5];
     const double* prim[6];  // rho,u,v,w,p,T
@@ -2469,6 +2495,13 @@ struct SensorArgs {
     const double* prs;
     double* ssf;
     unsigned char* lshock;
+    // k_grad_ssf: the velocity and the metric lines
+    const double* vel[3];
+    const double* xi[3];
+    // a two-dimensional step: the pressure of the planes k = -1 and 1 is
+    // that of the node (qswap copies it there; the copies are written only
+    // where a call ends)
+    int p2d;
 };
 
 // A bounded low / high end of an axis: ntype 1 / 2, and both ends of ntype
@@ -2479,23 +2512,18 @@ struct SensorArgs {
 __host__ __device__ __forceinline__ bool lo_end(int nt) { return nt == 1 || nt == 4; }
 __host__ __device__ __forceinline__ bool hi_end(int nt) { return nt == 2 || nt == 4; }
 
-// ducrossensor, part 1 (src/commcal.F90:236-272): ssf on 0..n; the
-// pressure stencil is clamped at a bounded end (ntype 1 and 2 in the
-// reference, both ends of ntype 4)
-__global__ void k_ducros_ssf(SensorArgs a)
+// ducrossensor, part 1 (src/commcal.F90:236-272), at one node from its
+// velocity gradients dv (3(m-1)+(n-1): dvel(m,n)); the pressure stencil is
+// clamped at a bounded end (ntype 1 and 2 in the reference, both ends of
+// ntype 4)
+__device__ __forceinline__ double ssf_of(const SensorArgs& a, int i, int j, int k, long gi,
+                                         const double* dv)
 {
-    const long p = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long ni = a.g.n[0] + 1, nj = a.g.n[1] + 1;
-    if (p >= ni * nj * (a.g.n[2] + 1)) return;
-    int i, j, k;
-    split3(p, ni, nj, i, j, k);
-    const long gi = gidx(a.g, i, j, k);
-    const double div = a.dvel[0][gi] + a.dvel[4][gi] + a.dvel[8][gi];
+    const double div = dv[0] + dv[4] + dv[8];
     const double div2 = div * div;
-    // dvel(m,n) is field 3(m-1)+(n-1)
-    const double vx = a.dvel[7][gi] - a.dvel[5][gi];  // dvel(3,2) - dvel(2,3)
-    const double vy = a.dvel[2][gi] - a.dvel[6][gi];  // dvel(1,3) - dvel(3,1)
-    const double vz = a.dvel[3][gi] - a.dvel[1][gi];  // dvel(2,1) - dvel(1,2)
+    const double vx = dv[7] - dv[5];  // dvel(3,2) - dvel(2,3)
+    const double vy = dv[2] - dv[6];  // dvel(1,3) - dvel(3,1)
+    const double vz = dv[3] - dv[1];  // dvel(2,1) - dvel(1,2)
     const double vort = vx * vx + vy * vy + vz * vz;
     int ip1 = i + 1, im1 = i - 1, jp1 = j + 1, jm1 = j - 1, kp1 = k + 1, km1 = k - 1;
     if (lo_end(a.ntype[0]) && im1 < 0) im1 = 0;
@@ -2508,45 +2536,37 @@ __global__ void k_ducros_ssf(SensorArgs a)
     const double* P = a.prs;
     const double pi1 = P[gidx(a.g, ip1, j, k)], pi0 = P[gidx(a.g, im1, j, k)];
     const double pj1 = P[gidx(a.g, i, jp1, k)], pj0 = P[gidx(a.g, i, jm1, k)];
-    const double pk1 = P[gidx(a.g, i, j, kp1)], pk0 = P[gidx(a.g, i, j, km1)];
+    const double pk1 = a.p2d ? pc : P[gidx(a.g, i, j, kp1)];
+    const double pk0 = a.p2d ? pc : P[gidx(a.g, i, j, km1)];
     const double dpdi = fabs(pi1 - 2.0 * pc + pi0) / (pi1 + 2.0 * pc + pi0);
     const double dpdj = fabs(pj1 - 2.0 * pc + pj0) / (pj1 + 2.0 * pc + pj0);
     const double dpdk = fabs(pk1 - 2.0 * pc + pk0) / (pk1 + 2.0 * pc + pk0);
-    a.ssf[gi] = div2 / (div2 + vort + 1.e-30) * uwd::max2(uwd::max2(dpdi, dpdj), dpdk);
+    return div2 / (div2 + vort + 1.e-30) * uwd::max2(uwd::max2(dpdi, dpdj), dpdk);
 }
 
-// dataswap(ssf) (src/commcal.F90:276; src/parallel.F90:4170-4175): a halo
-// cell takes the interior value at its periodically wrapped coordinates;
-// halo cells of non-periodic axes are zero (no neighbour on one domain).
-// Reads the interior, writes halo cells only.  A two-dimensional box needs
-// the plane k = 0 only: the window max skips the k axis there (the k halo
-// planes would repeat the plane itself, which the window already holds).
-__global__ void k_ssf_halo(SensorArgs a)
+__global__ void k_ducros_ssf(SensorArgs a)
 {
     const long p = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long ni = a.g.n[0] + 1 + 2 * HM, nj = a.g.n[1] + 1 + 2 * HM;
-    const long nk = a.ndims == 2 ? 1 : a.g.n[2] + 1 + 2 * HM;
-    if (p >= ni * nj * nk) return;
-    int c[3];
-    split3(p, ni, nj, c[0], c[1], c[2]);
-    c[0] -= HM;
-    c[1] -= HM;
-    c[2] = a.ndims == 2 ? 0 : c[2] - HM;
-    bool halo = false, keep = true;
-    int s[3];
-    for (int d = 0; d < 3; ++d) {
-        s[d] = c[d];
-        if (c[d] >= 0 && c[d] <= a.g.n[d]) continue;
-        halo = true;
-        if (d < a.ndims && a.ntype[d] == 3) s[d] = c[d] < 0 ? c[d] + a.g.n[d] : c[d] - a.g.n[d];
-        else keep = false;
-    }
-    if (!halo) return;
-    a.ssf[gidx(a.g, c[0], c[1], c[2])] = keep ? a.ssf[gidx(a.g, s[0], s[1], s[2])] : 0.0;
+    const long ni = a.g.n[0] + 1, nj = a.g.n[1] + 1;
+    if (p >= ni * nj * (a.g.n[2] + 1)) return;
+    int i, j, k;
+    split3(p, ni, nj, i, j, k);
+    const long gi = gidx(a.g, i, j, k);
+    double dv[9];
+#pragma unroll
+    for (int m = 0; m < 9; ++m) dv[m] = a.dvel[m][gi];
+    a.ssf[gi] = ssf_of(a, i, j, k, gi, dv);
 }
 
 // ducrossensor, part 2 (src/commcal.F90:278-316): lshock = max of ssf over
-// offsets -hm+1..hm along each axis > shkcrt, clamped at bounded ends
+// offsets -hm+1..hm along each axis > shkcrt, clamped at bounded ends;
+// along a periodic axis the offsets wrap (dataswap(ssf), src/commcal.F90:
+// 276, src/parallel.F90:4170-4175, which a two-dimensional box's k axis does
+// not need: its planes repeat the plane itself).
+// A node whose windows leave no end of the box, all but a frame of them,
+// reads them at fixed distances: with the clamp and the 64-bit index of
+// every offset the kernel was bound by its index arithmetic (555 vector
+// instructions a wavefront).
 __global__ void k_ducros_flag(SensorArgs a)
 {
     const long p = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -2554,17 +2574,30 @@ __global__ void k_ducros_flag(SensorArgs a)
     if (p >= ni * nj * (a.g.n[2] + 1)) return;
     int c0[3];
     split3(p, ni, nj, c0[0], c0[1], c0[2]);
+    const long gi = gidx(a.g, c0[0], c0[1], c0[2]);
     double m = 0.0;
-    for (int d = 0; d < a.ndims; ++d)
-        for (int o = -HM + 1; o <= HM; ++o) {
-            int c[3] = {c0[0], c0[1], c0[2]};
-            int t = c[d] + o;
-            if (lo_end(a.ntype[d]) && t < 0) t = 0;
-            if (hi_end(a.ntype[d]) && t > a.g.n[d]) t = a.g.n[d];
-            c[d] = t;
-            m = uwd::max2(m, a.ssf[gidx(a.g, c[0], c[1], c[2])]);
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        if (d >= a.ndims) break;
+        const int n = a.g.n[d];
+        const double* f = a.ssf + gi;
+        if (c0[d] >= HM - 1 && c0[d] + HM <= n) {
+            const int sd = (int)a.g.s[d];
+#pragma unroll
+            for (int o = -HM + 1; o <= HM; ++o) m = uwd::max2(m, f[o * sd]);
+        } else {
+            for (int o = -HM + 1; o <= HM; ++o) {
+                int t = c0[d] + o;
+                if (a.ntype[d] == 3) t = t < 0 ? t + n : (t > n ? t - n : t);
+                if (lo_end(a.ntype[d]) && t < 0) t = 0;
+                if (hi_end(a.ntype[d]) && t > n) t = n;
+                // (a rank's interface end, ntype 1's high and 2's low: the
+                // halo, which no neighbour fills on one domain, is zero)
+                m = uwd::max2(m, t < 0 || t > n ? 0.0 : f[(long)(t - c0[d]) * a.g.s[d]]);
+            }
         }
-    a.lshock[gidx(a.g, c0[0], c0[1], c0[2])] = m > a.shkcrt ? 1 : 0;
+    }
+    a.lshock[gi] = m > a.shkcrt ? 1 : 0;
 }
 
 struct GradXArgs {
@@ -2596,8 +2629,8 @@ __device__ __forceinline__ double diff6ec_at(const double* base, long stride, in
 // gradcal with the explicit 6th-order derivative (difschm '643e'),
 // src/comsolver.F90:244-497: dvel(m,d) = d/dxi_d(u_m) * dxi(d,d)
 // (streaming stores, as in k_rk: 2048^2 Riemann step 4.01 -> 3.89 ms; the
-// qrhs that k_zero_qrhs clears and k_uwd accumulates stays cached, which
-// measured 40 us per step faster than streaming it)
+// qrhs that k_uwd accumulates stays cached, which measured 40 us per step
+// faster than streaming it)
 __global__ void k_grad_explicit(GradXArgs a)
 {
     const long p = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -2622,6 +2655,35 @@ __global__ void k_grad_explicit(GradXArgs a)
             else st_nt(&a.dtmp[d][gi], df * x);
         }
     }
+}
+
+// The shock sensor's ssf from the velocity, without storing the gradients:
+// k_grad_explicit's velocity part, then k_ducros_ssf, at one node.  Whole
+// steps run it where nothing reads the gradients (the inviscid upwind
+// fluxes do not): 5 fields move instead of 27.
+__global__ __launch_bounds__(256) void k_grad_ssf(SensorArgs a)
+{
+    const long p = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long ni = a.g.n[0] + 1, nj = a.g.n[1] + 1;
+    if (p >= ni * nj * (a.g.n[2] + 1)) return;
+    int c[3];
+    split3(p, ni, nj, c[0], c[1], c[2]);
+    const long gi = gidx(a.g, c[0], c[1], c[2]);
+    double dv[9];
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        if (d >= a.ndims) {
+#pragma unroll
+            for (int m = 0; m < 3; ++m) dv[3 * m + d] = 0.0;
+            continue;
+        }
+        const long st = a.g.s[d];
+        const double x = a.xi[d][c[d] + HM];
+#pragma unroll
+        for (int m = 0; m < 3; ++m)
+            dv[3 * m + d] = diff6ec_at(a.vel[m] + gi - (long)c[d] * st, st, c[d], a.g.n[d], a.ntype[d]) * x;
+    }
+    a.ssf[gi] = ssf_of(a, c[0], c[1], c[2], gi, dv);
 }
 
 struct FieldXArgs {
@@ -2693,13 +2755,11 @@ __global__ void k_sw_field(CmpArgs a)
     for (int m = 0; m < 5; ++m) q[m] = a.q[m][gi];
     const double xv = a.xi[t + HM];
     const double dxi[3] = {a.dir == 0 ? xv : 0.0, a.dir == 1 ? xv : 0.0, a.dir == 2 ? xv : 0.0};
-    double fp[5], fm[5];
-    uwd::sw_split(a.gamma, a.mach, a.prim[0][gi], vel, a.prim[4][gi], a.prim[5][gi], q, dxi,
-                  a.jac[gi], fp, fm);
-    for (int m = 0; m < 5; ++m) {
-        a.sw[m][gi] = fp[m];
-        a.sw[5 + m][gi] = fm[m];
-    }
+    double f[10];
+    uwd::sw_split(a.gamma, a.mach, a.prim[0][gi], vel, a.prim[4][gi], a.prim[5][gi], q, dxi, xv,
+                  a.jac[gi], [&](int c, double v) { f[c] = v; });
+#pragma unroll
+    for (int m = 0; m < 10; ++m) a.sw[m][gi] = f[m];
 }
 
 // flux_compact (src/flux.F90:125-256) of one split-flux component along one
@@ -2806,18 +2866,6 @@ __global__ void k_recons_field(ReconsArgs a)
     a.fh[g0 + (long)i * st] = uwd::recons_exp(f8, i, dim, nte, a.recon, a.shock != 0, a.bfac);
 }
 
-// Zero qrhs on the interior (qrhs=0 before rhscal, src/mainloop.F90:404)
-__global__ void k_zero_qrhs(UwdArgs a)
-{
-    const long p = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long ni = a.g.n[0] + 1, nj = a.g.n[1] + 1;
-    if (p >= ni * nj * (a.g.n[2] + 1)) return;
-    int ci, cj, ck;
-    split3(p, ni, nj, ci, cj, ck);
-    const long gi = gidx(a.g, ci, cj, ck);
-    for (int m = 0; m < 5; ++m) a.qrhs[m][gi] = 0.0;
-}
-
 // convrsduwd along one axis, src/solver.F90:549-1202 (no species, crinod
 // false, no solids).  A tile is TL lines x S interfaces i0-1 .. i0+S-2:
 //  1. the Steger-Warming split fluxes of nodes i0-4 .. i0+S+2 (their index
@@ -2826,7 +2874,9 @@ __global__ void k_zero_qrhs(UwdArgs a)
 //     of F+ and F-, projected on the Roe eigenvectors where the scheme and
 //     the shock flag ask for it;
 //  3. qrhs(i) += Fh(i) - Fh(i-1) for the nodes i0 .. i0+S-2 within is..ie
-//     (negated on the last axis: qrhs=-qrhs, src/solver.F90:243).
+//     (from zero on the first axis: qrhs=0, src/mainloop.F90:404; negated on
+//     the last: qrhs=-qrhs, src/solver.F90:243).  Every axis covers the same
+//     nodes, and the others keep the zeros of the allocation.
 // x tiles are 1 line x 256 interfaces; y/z tiles 16 lines (consecutive i,
 // 128-byte rows) x 16 interfaces.
 // LD: the explicit path with MP7-LD (reschem 5), whose reconstruction needs
@@ -2835,12 +2885,16 @@ __global__ void k_zero_qrhs(UwdArgs a)
 // scratch cost less than the waves gained: MP7 at 2048^2 from 445 to 314 us
 // per launch).
 template <bool XD, bool CMP, bool LD = false>
-__global__ __launch_bounds__(256, CMP || LD ? 1 : 4) void k_uwd(UwdArgs a)
+__global__ __launch_bounds__(256, LD ? 3 : CMP ? 1 : 4) void k_uwd(UwdArgs a)
 {
     constexpr int TL = XD ? 1 : 16;
     constexpr int S = XD ? 256 : 16;
     constexpr int NN = S + 7;
-    __shared__ double sw[TL * NN * 10];
+    // component after component, the lines of a node side by side: the
+    // threads of a wavefront then read consecutive doubles (with the ten
+    // components of a node together they met in a quarter of the banks)
+    constexpr int NT = TL * NN;
+    __shared__ double sw[NT * 10];
     __shared__ double fh[TL * S * 5];
     const int tid = threadIdx.x;
     int bid = blockIdx.x;
@@ -2871,9 +2925,9 @@ __global__ __launch_bounds__(256, CMP || LD ? 1 : 4) void k_uwd(UwdArgs a)
         // run-time axis would live in scratch memory)
         const double xv = a.xi[node + HM];
         const double dxi[3] = {dir == 0 ? xv : 0.0, dir == 1 ? xv : 0.0, dir == 2 ? xv : 0.0};
-        double* o = sw + (l * NN + t) * 10;
+        double* o = sw + t * TL + l;
         uwd::sw_split(a.gamma, a.mach, a.prim[0][gi], vel, a.prim[4][gi], a.prim[5][gi], q, dxi,
-                      a.jac[gi], o, o + 5);
+                      xv, a.juni ? a.j0 : a.jac[gi], [&](int c, double v) { o[c * NT] = v; });
     }
     __syncthreads();
     // 2. interface fluxes
@@ -2906,7 +2960,7 @@ __global__ __launch_bounds__(256, CMP || LD ? 1 : 4) void k_uwd(UwdArgs a)
             r = uwd::roe_state(a.gamma, a.prim[0][gl], a.prim[4][gl], a.q[4][gl], vl, dl,
                                a.prim[0][gr], a.prim[4][gr], a.q[4][gr], vr, dr);
         }
-        const double* base = sw + l * NN * 10;
+        const double* base = sw + l;
         double fhc[5];
         if constexpr (CMP) {
             // convrsdcmp (src/solver.F90:1340-1460): 5-point stencils of
@@ -2927,18 +2981,20 @@ __global__ __launch_bounds__(256, CMP || LD ? 1 : 4) void k_uwd(UwdArgs a)
                     uwd::lev_row(r, m, lv);
 #pragma unroll
                     for (int w = 0; w < 5; ++w) {
-                        const double* P = base + (s + 1 + w) * 10;      // node ii+w-2
-                        const double* M = base + (s + 6 - w) * 10 + 5;  // node ii+3-w
-                        fp[w] = lv[0] * P[0] + lv[1] * P[1] + lv[2] * P[2] + lv[3] * P[3] + lv[4] * P[4];
-                        fm[w] = lv[0] * M[0] + lv[1] * M[1] + lv[2] * M[2] + lv[3] * M[3] + lv[4] * M[4];
+                        const double* P = base + (s + 1 + w) * TL;           // node ii+w-2
+                        const double* M = base + (s + 6 - w) * TL + 5 * NT;  // node ii+3-w
+                        fp[w] = lv[0] * P[0] + lv[1] * P[NT] + lv[2] * P[2 * NT] +
+                                lv[3] * P[3 * NT] + lv[4] * P[4 * NT];
+                        fm[w] = lv[0] * M[0] + lv[1] * M[NT] + lv[2] * M[2 * NT] +
+                                lv[3] * M[3 * NT] + lv[4] * M[4 * NT];
                     }
                     cpl = lv[0] * cp5[0] + lv[1] * cp5[1] + lv[2] * cp5[2] + lv[3] * cp5[3] + lv[4] * cp5[4];
                     cml = lv[0] * cm5[0] + lv[1] * cm5[1] + lv[2] * cm5[2] + lv[3] * cm5[3] + lv[4] * cm5[4];
                 } else {
 #pragma unroll
                     for (int w = 0; w < 5; ++w) {
-                        fp[w] = base[(s + 1 + w) * 10 + m];
-                        fm[w] = base[(s + 6 - w) * 10 + 5 + m];
+                        fp[w] = base[(s + 1 + w) * TL + m * NT];
+                        fm[w] = base[(s + 6 - w) * TL + (5 + m) * NT];
                     }
                     cpl = cp5[m];
                     cml = cm5[m];
@@ -2965,12 +3021,13 @@ __global__ __launch_bounds__(256, CMP || LD ? 1 : 4) void k_uwd(UwdArgs a)
                 if (chr) {
 #pragma unroll
                     for (int w = 0; w < 8; ++w) {
-                        const double* P = base + (s + w) * 10;  // node ii+w-3
-                        fp[w] = lv[0] * P[0] + lv[1] * P[1] + lv[2] * P[2] + lv[3] * P[3] + lv[4] * P[4];
+                        const double* P = base + (s + w) * TL;  // node ii+w-3
+                        fp[w] = lv[0] * P[0] + lv[1] * P[NT] + lv[2] * P[2 * NT] +
+                                lv[3] * P[3 * NT] + lv[4] * P[4 * NT];
                     }
                 } else {
 #pragma unroll
-                    for (int w = 0; w < 8; ++w) fp[w] = base[(s + w) * 10 + m];
+                    for (int w = 0; w < 8; ++w) fp[w] = base[(s + w) * TL + m * NT];
                 }
                 v1 = uwd::recons_exp<LD>(fp, ii, dim, nte, a.recon, lsh, a.bfac);
             }
@@ -2980,28 +3037,29 @@ __global__ __launch_bounds__(256, CMP || LD ? 1 : 4) void k_uwd(UwdArgs a)
                 if (chr) {
 #pragma unroll
                     for (int w = 0; w < 8; ++w) {
-                        const double* M = base + (s + 7 - w) * 10 + 5;  // node ii+4-w
-                        fm[w] = lv[0] * M[0] + lv[1] * M[1] + lv[2] * M[2] + lv[3] * M[3] + lv[4] * M[4];
+                        const double* M = base + (s + 7 - w) * TL + 5 * NT;  // node ii+4-w
+                        fm[w] = lv[0] * M[0] + lv[1] * M[NT] + lv[2] * M[2 * NT] +
+                                lv[3] * M[3 * NT] + lv[4] * M[4 * NT];
                     }
                 } else {
 #pragma unroll
-                    for (int w = 0; w < 8; ++w) fm[w] = base[(s + 7 - w) * 10 + 5 + m];
+                    for (int w = 0; w < 8; ++w) fm[w] = base[(s + 7 - w) * TL + (5 + m) * NT];
                 }
                 v2 = uwd::recons_exp<LD>(fm, ii, dim, nte, a.recon, lsh, a.bfac);
             }
             fhc[m] = v1 + v2;
         }
         }
-        double* F = fh + (l * S + s) * 5;
+        double* F = fh + s * TL + l;
         if (chr) {
             for (int m = 0; m < 5; ++m) {
                 double rv[5];
                 uwd::rev_row(r, m, rv);
-                F[m] = rv[0] * fhc[0] + rv[1] * fhc[1] + rv[2] * fhc[2] + rv[3] * fhc[3] +
+                F[m * TL * S] = rv[0] * fhc[0] + rv[1] * fhc[1] + rv[2] * fhc[2] + rv[3] * fhc[3] +
                        rv[4] * fhc[4];
             }
         } else {
-            for (int m = 0; m < 5; ++m) F[m] = fhc[m];
+            for (int m = 0; m < 5; ++m) F[m * TL * S] = fhc[m];
         }
     }
     __syncthreads();
@@ -3012,14 +3070,14 @@ __global__ __launch_bounds__(256, CMP || LD ? 1 : 4) void k_uwd(UwdArgs a)
         int i, j, k;
         line_node(l, node, i, j, k);
         const long gi = gidx(a.g, i, j, k);
-        const double* F1 = fh + (l * S + s) * 5;
-        const double* F0 = F1 - 5;
+        const double* F1 = fh + s * TL + l;
+        const double* F0 = F1 - TL;
         double qr[5];
 #pragma unroll
-        for (int m = 0; m < 5; ++m) qr[m] = a.qrhs[m][gi];
+        for (int m = 0; m < 5; ++m) qr[m] = a.first ? 0.0 : a.qrhs[m][gi];
 #pragma unroll
         for (int m = 0; m < 5; ++m) {
-            const double v = qr[m] + F1[m] - F0[m];
+            const double v = qr[m] + F1[m * TL * S] - F0[m * TL * S];
             a.qrhs[m][gi] = a.last ? -v : v;
         }
     }
@@ -4140,7 +4198,8 @@ int do_filterq(astr_ctx* c)
     return ASTR_OK;
 }
 
-int do_qswap(astr_ctx* c)
+// edge: a two-dimensional box whose primitives k_rk has just written from q
+int do_qswap(astr_ctx* c, bool edge = false)
 {
     PtArgs a = pt_args(c);
     const int n0 = c->g.n[0], n1 = c->g.n[1], n2 = c->g.n[2];
@@ -4152,6 +4211,7 @@ int do_qswap(astr_ctx* c)
             a.axis = d;
             TRY(launch_pt(c, k_qswap2d_line, (long)c->g.n[1 - d] + 1, a));
         }
+        if (edge) return launch_pt(c, k_qswap2d_edge, 2L * (n0 + 1 + n1 + 1), a);
         return launch_pt(c, k_qswap2d_plane, (long)(n0 + 1) * (n1 + 1), a);
     }
     // each part runs on a periodic axis only (the single-rank branches of
@@ -4383,8 +4443,9 @@ int do_grad_explicit(astr_ctx* c)
     return ASTR_OK;
 }
 
-// ducrossensor: ssf, its halo swap, the windowed flag
-int do_sensor(astr_ctx* c)
+// ducrossensor: ssf and the windowed flag.  fused: the velocity gradients
+// are formed on the way and not stored; p2d: see SensorArgs.
+int do_sensor(astr_ctx* c, bool fused = false, bool p2d = false)
 {
     SensorArgs a{};
     a.g = c->g;
@@ -4397,11 +4458,14 @@ int do_sensor(astr_ctx* c)
     a.prs = c->prim[4];
     a.ssf = c->ssf;
     a.lshock = c->lshock;
+    for (int m = 0; m < 3; ++m) {
+        a.vel[m] = c->prim[1 + m];
+        a.xi[m] = c->xi + m * c->xi_stride;
+    }
+    a.p2d = p2d;
     const long n = n_interior(c);
-    const long nh = a.ndims == 2 ? (long)(c->g.n[0] + 1 + 2 * HM) * (c->g.n[1] + 1 + 2 * HM)
-                                 : n_haloed(c);
-    hipLaunchKernelGGL(k_ducros_ssf, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, c->stream, a);
-    hipLaunchKernelGGL(k_ssf_halo, dim3((unsigned)((nh + 255) / 256)), dim3(256), 0, c->stream, a);
+    hipLaunchKernelGGL(fused ? k_grad_ssf : k_ducros_ssf, dim3((unsigned)((n + 255) / 256)),
+                       dim3(256), 0, c->stream, a);
     hipLaunchKernelGGL(k_ducros_flag, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, c->stream, a);
     HIPCHK(hipGetLastError());
     return ASTR_OK;
@@ -4438,10 +4502,9 @@ int do_upwind(astr_ctx* c)
     for (int m = 0; m < 5; ++m) { a.q[m] = c->q[m]; a.qrhs[m] = c->qrhs[m]; }
     for (int m = 0; m < 6; ++m) a.prim[m] = c->prim[m];
     a.jac = c->jac;
+    a.juni = c->juni;
+    a.j0 = c->j0;
     a.lshock = c->lshock;
-    const long n = n_interior(c);
-    hipLaunchKernelGGL(k_zero_qrhs, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, c->stream, a);
-    HIPCHK(hipGetLastError());
     for (int d = 0; d < nd; ++d) {
         a.dir = d;
         a.ntype = nts[d];
@@ -4455,6 +4518,7 @@ int do_upwind(astr_ctx* c)
         a.b0 = lo[ob];
         a.b1 = hi[ob];
         a.xi = c->xi + d * c->xi_stride;
+        a.first = d == 0;
         a.last = d == nd - 1;
         const int S = d == 0 ? 256 : 16, TL = d == 0 ? 1 : 16;
         a.ntile_line = (hi[d] - lo[d] + 1 + S - 2) / (S - 1);
@@ -4666,10 +4730,11 @@ int time_mark(astr_ctx* c, int slot)
 // step, so no qsave = q J is stored (5 fields per step fewer).  The
 // buffers then alternate from step to step; a generation bump makes a
 // batch that holds this context rebuild its launches.
-// last: no other step follows at once, so the x gradients of the last stage
-// are kept for the calls that read them (statistics, astr_download_rhs).
+// first, last: no other step of the same call comes before or after, so the
+// state a caller left is taken as it is, and what a later call reads
+// (gradients; 2-D: the pressure planes) is left in memory by the last stage.
 int do_step(astr_ctx* c, double dt, double* stats_slot, bool timed, bool alt = false,
-            bool last = true)
+            bool first = true, bool last = true)
 {
     c->bc_dt = dt;  // boucon's outflow reads the step's deltat
     // timing families: 0 filter, 1 boucon and qswap, 2 grad, 3 central:
@@ -4724,7 +4789,11 @@ int do_step(astr_ctx* c, double dt, double* stats_slot, bool timed, bool alt = f
         // boucon before qswap (src/mainloop.F90:413-415), at the step's
         // start time in every stage
         TRY(do_boucon(c));
-        TRY(do_qswap(c));
+        // (where a call begins or ends the whole plane: the primitives may
+        // not be q's yet, and the pressure planes are left for the host)
+        const bool ends = (s == 1 && first) || (s == 3 && last);
+        const bool edge = upwind && c->g.n[2] == 0 && !ends;
+        TRY(do_qswap(c, edge));
         if (timed) TRY(time_mark(c, 2));
         // rkfirst's statcal sees the stage-1 state and its gradients; the
         // central path sums it with the fluxes, which load the same inputs
@@ -4732,9 +4801,12 @@ int do_step(astr_ctx* c, double dt, double* stats_slot, bool timed, bool alt = f
             TRY(do_central_flux(c, s == 3 && last, s == 1 ? stats_slot : nullptr,
                                 timed ? 3 : -1));
         } else {
-            TRY(do_grad(c));
+            // the sensor alone reads the gradients of an inviscid upwind
+            // stage, unless they stay for the host or the statistics
+            const bool keep = !c->p.deriv_explicit || (s == 3 && last) || (s == 1 && stats_slot);
+            if (keep) TRY(do_grad(c));
             if (timed) TRY(time_mark(c, 3));
-            if (sensor_on(c)) TRY(do_sensor(c));
+            if (sensor_on(c)) TRY(do_sensor(c, !keep, edge));
         }
         if (timed) TRY(time_mark(c, 4));
         if (upwind && s == 1 && stats_slot) TRY(launch_stats(c, stats_slot));
@@ -6024,7 +6096,7 @@ static int rk3_steps(astr_ctx* c, int32_t nsteps, double dt, double* stats, bool
     for (int s = 0; s < nsteps; ++s) {
         const int slot = s - done;
         TRY(do_step(c, dt, stats ? c->stats_dev + 3 * slot : nullptr, c->timing == 1, true,
-                    s + 1 == nsteps));
+                    s == 0, s + 1 == nsteps));
         if (stats && (slot + 1 == STATS_SLOTS || s + 1 == nsteps)) {
             HIPCHK(hipMemcpyAsync(stats + 3 * (long)done, c->stats_dev,
                                   sizeof(double) * 3 * (slot + 1), hipMemcpyDeviceToHost,
@@ -6666,7 +6738,7 @@ int astr_adjoint_record(astr_ctx* c, int32_t nsteps, double dt, int32_t ckpt, do
         if (seg == nseg - 1) {
             TRY(segment_fwd(c, nstates, 3 * (t1 - t0), dt));
         } else {
-            for (long t = t0; t < t1; ++t) TRY(do_step(c, dt, nullptr, false, true, false));
+            for (long t = t0; t < t1; ++t) TRY(do_step(c, dt, nullptr, false, true, true, false));
         }
     }
     TRY(save_state(c, nseg));

@@ -254,29 +254,33 @@ __device__ double recons_exp(const double* f, int inode, int dim, int ntype, int
 }
 
 // flux_steger_warming at one node, src/riemann.F90:23-161 (no species);
-// sos = sqrt(T)/Ma (src/fludyna.F90:832-859)
-__device__ void sw_split(double gamma, double mach, double rho, const double* vel, double prs,
-                         double tmp, const double* q, const double* dxi, double jacob, double* fp,
-                         double* fm)
+// sos = sqrt(T)/Ma (src/fludyna.F90:832-859).  dxi has one component xv off
+// zero (rectilinear metrics), so the reference's 1/sqrt(dxi.dxi) is 1/|xv|
+// exactly: the square root of a rounded square is its argument's magnitude.
+// put(c, v) takes the components, c = 0..4 of F+ and 5..9 of F-.
+template <class O>
+__device__ __forceinline__ void sw_split(double gamma, double mach, double rho, const double* vel,
+                                         double prs, double tmp, const double* q,
+                                         const double* dxi, double xv, double jacob, const O& put)
 {
     const double eps = 0.04;
     const double uu = dxi[0] * vel[0] + dxi[1] * vel[1] + dxi[2] * vel[2];
-    const double var0 = 1.0 / sqrt(dxi[0] * dxi[0] + dxi[1] * dxi[1] + dxi[2] * dxi[2]);
+    const double var0 = 1.0 / fabs(xv);
     const double gpd0 = dxi[0] * var0, gpd1 = dxi[1] * var0, gpd2 = dxi[2] * var0;
     const double gm2 = 0.5 / gamma;
     const double css = sqrt(tmp) / mach;
     const double csa = css / var0;
     const double lmach = uu / csa;
     if (lmach >= 1.0 || lmach <= -1.0) {
-        double* f = lmach >= 1.0 ? fp : fm;
-        double* z = lmach >= 1.0 ? fm : fp;
-        f[0] = jacob * q[0] * uu;
-        f[1] = jacob * (q[1] * uu + dxi[0] * prs);
-        f[2] = jacob * (q[2] * uu + dxi[1] * prs);
-        f[3] = jacob * (q[3] * uu + dxi[2] * prs);
-        f[4] = jacob * (q[4] + prs) * uu;
+        const double f[5] = {jacob * q[0] * uu, jacob * (q[1] * uu + dxi[0] * prs),
+                             jacob * (q[2] * uu + dxi[1] * prs),
+                             jacob * (q[3] * uu + dxi[2] * prs), jacob * (q[4] + prs) * uu};
+        const bool pos = lmach >= 1.0;
 #pragma unroll
-        for (int k = 0; k < 5; ++k) z[k] = 0.0;
+        for (int k = 0; k < 5; ++k) {
+            put(k, pos ? f[k] : 0.0);
+            put(5 + k, pos ? 0.0 : f[k]);
+        }
         return;
     }
     const double l0 = uu, l3 = uu + csa, l4 = uu - csa;
@@ -290,17 +294,17 @@ __device__ void sw_split(double gamma, double mach, double rho, const double* ve
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
         const double* l = s == 0 ? lp : lm;
-        double* f = s == 0 ? fp : fm;
+        const int c = 5 * s;
         const double var1 = l[0];
         const double var2 = l[1] - l[2];
         const double var3 = 2.0 * l[0] - l[1] - l[2];
         const double var4 = var1 - var3 * gm2;
-        f[0] = jro * var4;
-        f[1] = jro * (var4 * vel[0] + var2 * css * gpd0 * gm2);
-        f[2] = jro * (var4 * vel[1] + var2 * css * gpd1 * gm2);
-        f[3] = jro * (var4 * vel[2] + var2 * css * gpd2 * gm2);
-        f[4] = jacob * (var1 * q[4] + rho * (var2 * uu * var0 * css * gm2 -
-                                             var3 * (fhi + css * css) * gm2 / (gamma - 1.0)));
+        put(c, jro * var4);
+        put(c + 1, jro * (var4 * vel[0] + var2 * css * gpd0 * gm2));
+        put(c + 2, jro * (var4 * vel[1] + var2 * css * gpd1 * gm2));
+        put(c + 3, jro * (var4 * vel[2] + var2 * css * gpd2 * gm2));
+        put(c + 4, jacob * (var1 * q[4] + rho * (var2 * uu * var0 * css * gm2 -
+                                                 var3 * (fhi + css * css) * gm2 / (gamma - 1.0))));
     }
 }
 
