@@ -37,6 +37,7 @@
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/astr_hip.h"
@@ -1101,6 +1102,7 @@ __global__ void k_qswap2d_plane(PtArgs a)
 // The same within a step: k_rk has just written the primitives of every
 // node from its q, so only the nodes that boucon set since, those of the
 // edges i = 0, n and j = 0, n, are refreshed.
+// (1025^2: 24 -> 5 us.)
 __global__ void k_qswap2d_edge(PtArgs a)
 {
     const int ni = a.g.n[0] + 1, nj = a.g.n[1] + 1;
@@ -2661,6 +2663,7 @@ __global__ void k_grad_explicit(GradXArgs a)
 // k_grad_explicit's velocity part, then k_ducros_ssf, at one node.  Whole
 // steps run it where nothing reads the gradients (the inviscid upwind
 // fluxes do not): 5 fields move instead of 27.
+// (k_grad_explicit + k_ducros_ssf -> this: 1025^2 80 -> 35 us, 96^3 85 -> 41.)
 __global__ __launch_bounds__(256) void k_grad_ssf(SensorArgs a)
 {
     const long p = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -2863,7 +2866,20 @@ __global__ void k_recons_field(ReconsArgs a)
 #pragma unroll
     for (int w = 0; w < 8; ++w) f8[w] = a.f[g0 + (long)(a.plus ? i - 3 + w : i + 4 - w) * st];
     const int nte = a.ntype == 4 ? (i < dim / 2 ? 1 : 2) : a.ntype;
-    a.fh[g0 + (long)i * st] = uwd::recons_exp(f8, i, dim, nte, a.recon, a.shock != 0, a.bfac);
+    auto go = [&](auto rs) {
+        return uwd::recons_exp<decltype(rs)::value>(f8, i, dim, nte, a.shock != 0, a.bfac);
+    };
+    double v;
+    switch (a.recon) {
+    case -1: v = go(std::integral_constant<int, -1>()); break;
+    case 0: v = go(std::integral_constant<int, 0>()); break;
+    case 1: v = go(std::integral_constant<int, 1>()); break;
+    case 2: v = go(std::integral_constant<int, 2>()); break;
+    case 3: v = go(std::integral_constant<int, 3>()); break;
+    case 5: v = go(std::integral_constant<int, 5>()); break;
+    default: v = go(std::integral_constant<int, 6>()); break;
+    }
+    a.fh[g0 + (long)i * st] = v;
 }
 
 // convrsduwd along one axis, src/solver.F90:549-1202 (no species, crinod
@@ -2877,26 +2893,50 @@ __global__ void k_recons_field(ReconsArgs a)
 //     (from zero on the first axis: qrhs=0, src/mainloop.F90:404; negated on
 //     the last: qrhs=-qrhs, src/solver.F90:243).  Every axis covers the same
 //     nodes, and the others keep the zeros of the allocation.
-// x tiles are 1 line x 256 interfaces; y/z tiles 16 lines (consecutive i,
+// x tiles are 4 lines x 64 interfaces; y/z tiles 16 lines (consecutive i,
 // 128-byte rows) x 16 interfaces.
-// LD: the explicit path with MP7-LD (reschem 5), whose reconstruction needs
-// 236 registers (2 waves per SIMD).  The other explicit schemes run with 4
-// waves per SIMD (128 registers; the dozen the compiler then keeps in
-// scratch cost less than the waves gained: MP7 at 2048^2 from 445 to 314 us
-// per launch).
-template <bool XD, bool CMP, bool LD = false>
-__global__ __launch_bounds__(256, LD ? 3 : CMP ? 1 : 4) void k_uwd(UwdArgs a)
+// RS: the explicit path's scheme (reschem), UWD_CMP convrsdcmp: with all of
+// them in one kernel the one with the most registers sets the occupancy of
+// every other.  MP7-LD runs with 3 waves per SIMD, the other explicit schemes
+// with 4.
+// Latency bound: a wave's chain of square roots, divisions and limiter
+// branches at 16 waves a CU.  x and y launches, MP7 with the sensor, in us:
+//                                                401x337      1025^2
+//   one kernel for all schemes                  29.7  32.7   94    97
+//   a kernel per scheme; where no interface
+//   is projected both stencils in flight        29.2  26.7   80    82
+//   x tiles of 4 lines, projections packed      23.1  26.5   64    84
+// A tile's projected interfaces (the flagged ones: a few per cent on the
+// Riemann problem) cost 13 us of the 29 at 401x337 while each sat on its own
+// thread, five fields in a row.
+constexpr int UWD_CMP = 100;
+// Interfaces per tile, S - 1 nodes' worth.  Along x 64 rather than 256 (one
+// line a tile): a line of 96 nodes left 158 of 256 threads idle (96^3, x: 130
+// -> 90 us; 1025^2: 80 -> 77).  Along y 32 (512 threads) measured 79 against
+// 82 us at 1025^2 and 29.6 against 26.7 at 401x337: 16.
+constexpr int UWD_SX = 64, UWD_SY = 16;
+template <bool XD, int RS>
+__global__ __launch_bounds__(256, RS == UWD_CMP ? 2 : RS == 5 ? 3 : 4) void k_uwd(UwdArgs a)
 {
-    constexpr int TL = XD ? 1 : 16;
-    constexpr int S = XD ? 256 : 16;
+    constexpr bool CMP = RS == UWD_CMP;
+    constexpr int S = XD ? UWD_SX : UWD_SY;
+    constexpr int TL = 256 / S;
     constexpr int NN = S + 7;
-    // component after component, the lines of a node side by side: the
-    // threads of a wavefront then read consecutive doubles (with the ten
-    // components of a node together they met in a quarter of the banks)
+    // component after component, along x the nodes of a line and along y and
+    // z the lines of a node side by side: the threads of a wavefront read
+    // consecutive doubles (with the ten components of a node together they
+    // met in a quarter of the banks)
     constexpr int NT = TL * NN;
+    constexpr int ST = XD ? 1 : TL;        // from a node to the next
+    constexpr int SL = XD ? NN : 1;        // from a line to the next
+    constexpr int FL = XD ? S : 1;         // the same of the interface fluxes
     __shared__ double sw[NT * 10];
     __shared__ double fh[TL * S * 5];
+    // the tile's projected interfaces (their threads' numbers)
+    __shared__ unsigned char flist[CMP ? 1 : 256];
+    __shared__ int nflag;
     const int tid = threadIdx.x;
+    if (!CMP && tid == 0) nflag = 0;
     int bid = blockIdx.x;
     const int seg = bid % a.ntile_line;
     bid /= a.ntile_line;
@@ -2912,8 +2952,8 @@ __global__ __launch_bounds__(256, LD ? 3 : CMP ? 1 : 4) void k_uwd(UwdArgs a)
         else { i = av; j = b; k = t; }
     };
     // 1. split fluxes
-    for (int e = tid; e < TL * NN; e += 256) {
-        const int l = e % TL, t = e / TL;
+    for (int e = tid; e < NT; e += 256) {
+        const int l = XD ? e / NN : e % TL, t = XD ? e % NN : e / TL;
         const int node = min(max(i0 - 4 + t, a.iss), a.iee);
         int i, j, k;
         line_node(l, node, i, j, k);
@@ -2925,44 +2965,53 @@ __global__ __launch_bounds__(256, LD ? 3 : CMP ? 1 : 4) void k_uwd(UwdArgs a)
         // run-time axis would live in scratch memory)
         const double xv = a.xi[node + HM];
         const double dxi[3] = {dir == 0 ? xv : 0.0, dir == 1 ? xv : 0.0, dir == 2 ? xv : 0.0};
-        double* o = sw + t * TL + l;
+        double* o = sw + t * ST + l * SL;
         uwd::sw_split(a.gamma, a.mach, a.prim[0][gi], vel, a.prim[4][gi], a.prim[5][gi], q, dxi,
                       xv, a.juni ? a.j0 : a.jac[gi], [&](int c, double v) { o[c * NT] = v; });
     }
     __syncthreads();
     // 2. interface fluxes
-    const int l = XD ? 0 : (tid & 15);
-    const int s = XD ? tid : (tid >> 4);
+    const int l = XD ? tid / S : (tid & 15);
+    const int s = XD ? tid % S : (tid >> 4);
     const int ii = i0 - 1 + s;  // interface ii+1/2
-    if (ii <= a.hi) {
-        bool lsh = true;
-        if (a.sensor) {
-            int i, j, k;
-            line_node(l, ii < 0 ? ii + 1 : ii, i, j, k);
-            const bool s1 = a.lshock[gidx(a.g, i, j, k)] != 0;
-            line_node(l, ii + 1 > dim ? ii : ii + 1, i, j, k);
-            lsh = s1 || a.lshock[gidx(a.g, i, j, k)] != 0;
-        }
-        // convrsdcmp projects every interface, convrsduwd only flagged ones
-        const bool chr = a.lchar && (CMP || lsh);
-        uwd::Roe r;
-        if (chr) {
-            int i, j, k;
-            line_node(l, ii, i, j, k);
-            const long gl = gidx(a.g, i, j, k);
-            line_node(l, ii + 1, i, j, k);
-            const long gr = gidx(a.g, i, j, k);
-            const double vl[3] = {a.prim[1][gl], a.prim[2][gl], a.prim[3][gl]};
-            const double vr[3] = {a.prim[1][gr], a.prim[2][gr], a.prim[3][gr]};
-            const double xl = a.xi[ii + HM], xr = a.xi[ii + 1 + HM];
-            const double dl[3] = {dir == 0 ? xl : 0.0, dir == 1 ? xl : 0.0, dir == 2 ? xl : 0.0};
-            const double dr[3] = {dir == 0 ? xr : 0.0, dir == 1 ? xr : 0.0, dir == 2 ? xr : 0.0};
-            r = uwd::roe_state(a.gamma, a.prim[0][gl], a.prim[4][gl], a.q[4][gl], vl, dl,
-                               a.prim[0][gr], a.prim[4][gr], a.q[4][gr], vr, dr);
-        }
-        const double* base = sw + l;
-        double fhc[5];
-        if constexpr (CMP) {
+    const bool act = ii <= a.hi;
+    bool lsh = true;
+    if (act && a.sensor) {
+        int i, j, k;
+        line_node(l, ii < 0 ? ii + 1 : ii, i, j, k);
+        const bool s1 = a.lshock[gidx(a.g, i, j, k)] != 0;
+        line_node(l, ii + 1 > dim ? ii : ii + 1, i, j, k);
+        lsh = s1 || a.lshock[gidx(a.g, i, j, k)] != 0;
+    }
+    // convrsdcmp projects every interface, convrsduwd only flagged ones
+    const bool chr = a.lchar && (CMP || lsh);
+    // the Roe state of interface ii+1/2 of line l
+    auto roe_at = [&](int l, int ii) {
+        int i, j, k;
+        line_node(l, ii, i, j, k);
+        const long gl = gidx(a.g, i, j, k);
+        line_node(l, ii + 1, i, j, k);
+        const long gr = gidx(a.g, i, j, k);
+        const double vl[3] = {a.prim[1][gl], a.prim[2][gl], a.prim[3][gl]};
+        const double vr[3] = {a.prim[1][gr], a.prim[2][gr], a.prim[3][gr]};
+        const double xl = a.xi[ii + HM], xr = a.xi[ii + 1 + HM];
+        const double dl[3] = {dir == 0 ? xl : 0.0, dir == 1 ? xl : 0.0, dir == 2 ? xl : 0.0};
+        const double dr[3] = {dir == 0 ? xr : 0.0, dir == 1 ? xr : 0.0, dir == 2 ? xr : 0.0};
+        return uwd::roe_state(a.gamma, a.prim[0][gl], a.prim[4][gl], a.q[4][gl], vl, dl,
+                              a.prim[0][gr], a.prim[4][gr], a.q[4][gr], vr, dr);
+    };
+    // recons_exp sees ntype 4 as ntype 1 on the low half of the line and
+    // ntype 2 on the high half: what the reference computes with the axis
+    // split over several ranks (the explicit flux has no closure at a rank
+    // interface)
+    auto closure = [&](int ii) { return a.ntype == 4 ? (ii < dim / 2 ? 1 : 2) : a.ntype; };
+    if constexpr (CMP) {
+        if (act) {
+            const double* base = sw + l * SL;
+            double* F = fh + s * ST + l * FL;
+            uwd::Roe r;
+            if (chr) r = roe_at(l, ii);
+            double fhc[5];
             // convrsdcmp (src/solver.F90:1340-1460): 5-point stencils of
             // iwind6 about the compact interface values, then mplimiter
             int i, j, k;
@@ -2981,8 +3030,8 @@ __global__ __launch_bounds__(256, LD ? 3 : CMP ? 1 : 4) void k_uwd(UwdArgs a)
                     uwd::lev_row(r, m, lv);
 #pragma unroll
                     for (int w = 0; w < 5; ++w) {
-                        const double* P = base + (s + 1 + w) * TL;           // node ii+w-2
-                        const double* M = base + (s + 6 - w) * TL + 5 * NT;  // node ii+3-w
+                        const double* P = base + (s + 1 + w) * ST;           // node ii+w-2
+                        const double* M = base + (s + 6 - w) * ST + 5 * NT;  // node ii+3-w
                         fp[w] = lv[0] * P[0] + lv[1] * P[NT] + lv[2] * P[2 * NT] +
                                 lv[3] * P[3 * NT] + lv[4] * P[4 * NT];
                         fm[w] = lv[0] * M[0] + lv[1] * M[NT] + lv[2] * M[2 * NT] +
@@ -2993,8 +3042,8 @@ __global__ __launch_bounds__(256, LD ? 3 : CMP ? 1 : 4) void k_uwd(UwdArgs a)
                 } else {
 #pragma unroll
                     for (int w = 0; w < 5; ++w) {
-                        fp[w] = base[(s + 1 + w) * TL + m * NT];
-                        fm[w] = base[(s + 6 - w) * TL + (5 + m) * NT];
+                        fp[w] = base[(s + 1 + w) * ST + m * NT];
+                        fm[w] = base[(s + 6 - w) * ST + (5 + m) * NT];
                     }
                     cpl = cp5[m];
                     cml = cm5[m];
@@ -3003,75 +3052,118 @@ __global__ __launch_bounds__(256, LD ? 3 : CMP ? 1 : 4) void k_uwd(UwdArgs a)
                 const double v2 = uwd::mplimiter(fm, cml, lsh, ii, dim, a.ntype);
                 fhc[m] = v1 + v2;
             }
-        } else {
-        // recons_exp sees ntype 4 as ntype 1 on the low half of the line
-        // and ntype 2 on the high half: what the reference computes with
-        // the axis split over several ranks (the explicit flux has no
-        // closure at a rank interface)
-        const int nte = a.ntype == 4 ? (ii < dim / 2 ? 1 : 2) : a.ntype;
-        for (int m = 0; m < 5; ++m) {
-            // the F+ stencil and its reconstruction, then F-'s: the empty
-            // asm keeps the second's LDS reads after the first's result, so
-            // that the two stencils are not live at once
-            double lv[5];
-            if (chr) uwd::lev_row(r, m, lv);
-            double v1, v2;
-            {
-                double fp[8];
-                if (chr) {
+            if (chr) {
+                for (int m = 0; m < 5; ++m) {
+                    double rv[5];
+                    uwd::rev_row(r, m, rv);
+                    F[m * TL * S] = rv[0] * fhc[0] + rv[1] * fhc[1] + rv[2] * fhc[2] +
+                                    rv[3] * fhc[3] + rv[4] * fhc[4];
+                }
+            } else {
+                for (int m = 0; m < 5; ++m) F[m * TL * S] = fhc[m];
+            }
+        }
+    } else {
+        // interfaces without a projection, nearly all of them: no Roe state
+        // to hold, so both stencils are in flight at once
+        if (act && !chr) {
+            const int nte = closure(ii);
+#pragma unroll 1
+            for (int m = 0; m < 5; ++m) {
+                const double* P = sw + l * SL + s * ST + m * NT;              // node ii-3
+                const double* M = sw + l * SL + (s + 7) * ST + (5 + m) * NT;  // node ii+4
+                double fp[8], fm[8];
+#pragma unroll
+                for (int w = 0; w < 8; ++w) {
+                    fp[w] = P[w * ST];
+                    fm[w] = M[-w * ST];
+                }
+                const double v1 = uwd::recons_exp<RS>(fp, ii, dim, nte, lsh, a.bfac);
+                const double v2 = uwd::recons_exp<RS>(fm, ii, dim, nte, lsh, a.bfac);
+                fh[s * ST + l * FL + m * TL * S] = v1 + v2;
+            }
+        }
+        if (act && chr) flist[atomicAdd(&nflag, 1)] = (unsigned char)tid;
+        __syncthreads();
+        // The projected interfaces, packed onto the tile's first threads: as
+        // many threads to an interface as the tile has (one, two, three or
+        // five), each taking its share of the five characteristic fields and
+        // forming the Roe state itself, so that the tile waits for one
+        // field's chain rather than five in a row.
+        const int nf = nflag;
+        const int share = nf <= 51 ? 1 : nf <= 85 ? 2 : nf <= 128 ? 3 : 5;
+        const int part = nf > 0 ? tid / nf : 5;
+        const int m0 = part * share, m1 = min(m0 + share, 5);
+        const bool mine = m0 < 5;
+        const int it = mine ? flist[tid - part * nf] : tid;
+        const int l2 = XD ? it / S : (it & 15), s2 = XD ? it % S : (it >> 4);
+        const int i2 = i0 - 1 + s2;
+        double* const F = fh + s2 * ST + l2 * FL;
+        uwd::Roe r;
+        double f[5];
+        if (mine) {
+            r = roe_at(l2, i2);
+            const double* base = sw + l2 * SL + s2 * ST;
+            const int nte = closure(i2);
+#pragma unroll 1
+            for (int m = m0; m < m1; ++m) {
+                // the F+ stencil and its reconstruction, then F-'s: the empty
+                // asm keeps the second's LDS reads after the first's result,
+                // so that the two stencils are not live at once
+                double lv[5], v1, v2;
+                uwd::lev_row(r, m, lv);
+                {
+                    double fp[8];
 #pragma unroll
                     for (int w = 0; w < 8; ++w) {
-                        const double* P = base + (s + w) * TL;  // node ii+w-3
+                        const double* P = base + w * ST;  // node ii+w-3
                         fp[w] = lv[0] * P[0] + lv[1] * P[NT] + lv[2] * P[2 * NT] +
                                 lv[3] * P[3 * NT] + lv[4] * P[4 * NT];
                     }
-                } else {
-#pragma unroll
-                    for (int w = 0; w < 8; ++w) fp[w] = base[(s + w) * TL + m * NT];
+                    v1 = uwd::recons_exp<RS>(fp, i2, dim, nte, true, a.bfac);
                 }
-                v1 = uwd::recons_exp<LD>(fp, ii, dim, nte, a.recon, lsh, a.bfac);
-            }
-            asm volatile("" : "+v"(v1) : : "memory");
-            {
-                double fm[8];
-                if (chr) {
+                asm volatile("" : "+v"(v1) : : "memory");
+                {
+                    double fm[8];
 #pragma unroll
                     for (int w = 0; w < 8; ++w) {
-                        const double* M = base + (s + 7 - w) * TL + 5 * NT;  // node ii+4-w
+                        const double* M = base + (7 - w) * ST + 5 * NT;  // node ii+4-w
                         fm[w] = lv[0] * M[0] + lv[1] * M[NT] + lv[2] * M[2 * NT] +
                                 lv[3] * M[3 * NT] + lv[4] * M[4 * NT];
                     }
-                } else {
-#pragma unroll
-                    for (int w = 0; w < 8; ++w) fm[w] = base[(s + 7 - w) * TL + (5 + m) * NT];
+                    v2 = uwd::recons_exp<RS>(fm, i2, dim, nte, true, a.bfac);
                 }
-                v2 = uwd::recons_exp<LD>(fm, ii, dim, nte, a.recon, lsh, a.bfac);
+                F[m * TL * S] = v1 + v2;
             }
-            fhc[m] = v1 + v2;
         }
+        // back to the conserved variables: every field of the interface is
+        // read before any of its fluxes is written
+        if (nf > 0) __syncthreads();
+        if (mine) {
+#pragma unroll
+            for (int m = 0; m < 5; ++m) f[m] = F[m * TL * S];
         }
-        double* F = fh + s * TL + l;
-        if (chr) {
-            for (int m = 0; m < 5; ++m) {
+        if (nf > 0) __syncthreads();
+        if (mine) {
+#pragma unroll 1
+            for (int m = m0; m < m1; ++m) {
                 double rv[5];
                 uwd::rev_row(r, m, rv);
-                F[m * TL * S] = rv[0] * fhc[0] + rv[1] * fhc[1] + rv[2] * fhc[2] + rv[3] * fhc[3] +
-                       rv[4] * fhc[4];
+                F[m * TL * S] =
+                    rv[0] * f[0] + rv[1] * f[1] + rv[2] * f[2] + rv[3] * f[3] + rv[4] * f[4];
             }
-        } else {
-            for (int m = 0; m < 5; ++m) F[m * TL * S] = fhc[m];
         }
     }
     __syncthreads();
     // 3. flux difference
     const int node = i0 - 1 + s;
-    const bool lvalid = XD || (a.a0 + ta * TL + l <= a.a1);
+    const bool lvalid = a.a0 + ta * TL + l <= a.a1;
     if (s >= 1 && node <= a.hi && lvalid) {
         int i, j, k;
         line_node(l, node, i, j, k);
         const long gi = gidx(a.g, i, j, k);
-        const double* F1 = fh + s * TL + l;
-        const double* F0 = F1 - TL;
+        const double* F1 = fh + s * ST + l * FL;
+        const double* F0 = F1 - ST;
         double qr[5];
 #pragma unroll
         for (int m = 0; m < 5; ++m) qr[m] = a.first ? 0.0 : a.qrhs[m][gi];
@@ -4480,6 +4572,20 @@ void uwd_range(int ntype, int n, int& lo, int& hi)
     hi = (ntype == 2 || ntype == 4) ? n - 1 : n;
 }
 
+template <int RS>
+void launch_uwd(astr_ctx* c, UwdArgs& a)
+{
+    const int m = a.hi - a.lo + 1;
+    const int S = a.dir == 0 ? UWD_SX : UWD_SY, TL = 256 / S;
+    a.ntile_line = (m + S - 2) / (S - 1);
+    a.ntile_a = (a.a1 - a.a0 + 1 + TL - 1) / TL;
+    const dim3 grid((unsigned)((long)a.ntile_line * a.ntile_a * (a.b1 - a.b0 + 1)));
+    if (a.dir == 0)
+        hipLaunchKernelGGL((k_uwd<true, RS>), grid, dim3(256), 0, c->stream, a);
+    else
+        hipLaunchKernelGGL((k_uwd<false, RS>), grid, dim3(256), 0, c->stream, a);
+}
+
 // qrhs=0, then convrsduwd (convection 1) or convrsdcmp (convection 2)
 // along each axis, the last one negating
 int do_upwind(astr_ctx* c)
@@ -4520,11 +4626,6 @@ int do_upwind(astr_ctx* c)
         a.xi = c->xi + d * c->xi_stride;
         a.first = d == 0;
         a.last = d == nd - 1;
-        const int S = d == 0 ? 256 : 16, TL = d == 0 ? 1 : 16;
-        a.ntile_line = (hi[d] - lo[d] + 1 + S - 2) / (S - 1);
-        a.ntile_a = (a.a1 - a.a0 + 1 + TL - 1) / TL;
-        const long nblk = (long)a.ntile_line * a.ntile_a * (a.b1 - a.b0 + 1);
-        if (nblk <= 0) continue;
         if (cmp) {
             // split fluxes and their compact interface fluxes first
             CmpArgs ca{};
@@ -4567,20 +4668,17 @@ int do_upwind(astr_ctx* c)
                 a.fhp[m] = c->fhf[m];
                 a.fhm[m] = c->fhf[5 + m];
             }
-            if (d == 0)
-                hipLaunchKernelGGL((k_uwd<true, true>), dim3((unsigned)nblk), dim3(256), 0, c->stream, a);
-            else
-                hipLaunchKernelGGL((k_uwd<false, true>), dim3((unsigned)nblk), dim3(256), 0, c->stream, a);
+            launch_uwd<UWD_CMP>(c, a);
         } else {
-            const bool ld = c->p.recon_schem == 5;
-            if (d == 0 && ld)
-                hipLaunchKernelGGL((k_uwd<true, false, true>), dim3((unsigned)nblk), dim3(256), 0, c->stream, a);
-            else if (d == 0)
-                hipLaunchKernelGGL((k_uwd<true, false>), dim3((unsigned)nblk), dim3(256), 0, c->stream, a);
-            else if (ld)
-                hipLaunchKernelGGL((k_uwd<false, false, true>), dim3((unsigned)nblk), dim3(256), 0, c->stream, a);
-            else
-                hipLaunchKernelGGL((k_uwd<false, false>), dim3((unsigned)nblk), dim3(256), 0, c->stream, a);
+            switch (c->p.recon_schem) {
+            case -1: launch_uwd<-1>(c, a); break;
+            case 0: launch_uwd<0>(c, a); break;
+            case 1: launch_uwd<1>(c, a); break;
+            case 2: launch_uwd<2>(c, a); break;
+            case 3: launch_uwd<3>(c, a); break;
+            case 5: launch_uwd<5>(c, a); break;
+            default: launch_uwd<6>(c, a); break;
+            }
         }
         HIPCHK(hipGetLastError());
     }

@@ -53,7 +53,7 @@ __device__ __forceinline__ double suw7(const double* u)
 
 // Suresh-Huynh monotonicity-preserving bounds on u(i-2..i+2) = u[0..4]
 // around the linear value, src/flux.F90:465-490
-__device__ double mp_limit(const double* u, double ul)
+__device__ __forceinline__ double mp_limit(const double* u, double ul)
 {
     const double dm1 = u[0] - 2.0 * u[1] + u[2];
     const double d0 = u[1] - 2.0 * u[2] + u[3];
@@ -70,7 +70,7 @@ __device__ double mp_limit(const double* u, double ul)
 }
 
 // MP5 without the optional arguments, src/flux.F90:434-496
-__device__ double mp5(const double* u)
+__device__ __forceinline__ double mp5(const double* u)
 {
     const double ul = suw5(u);
     const double uMP = u[2] + minmod2(u[3] - u[2], 4.0 * (u[2] - u[1]));
@@ -80,7 +80,7 @@ __device__ double mp5(const double* u)
 
 // MP5 with a supplied linear value and shock switch, and mplimiter,
 // src/flux.F90:363-379,434-496
-__device__ double mplimiter(const double* u, double ul, bool lskt, int inode, int dim, int ntype)
+__device__ __forceinline__ double mplimiter(const double* u, double ul, bool lskt, int inode, int dim, int ntype)
 {
     if ((ntype == 1 && (inode == 0 || inode == 1)) ||
         (ntype == 2 && (inode == dim - 1 || inode == dim - 2)))
@@ -91,7 +91,7 @@ __device__ double mplimiter(const double* u, double ul, bool lskt, int inode, in
 }
 
 // MP7, src/flux.F90:498-551
-__device__ double mp7(const double* u)
+__device__ __forceinline__ double mp7(const double* u)
 {
     const double ul = suw7(u);
     const double uMP = u[3] + minmod2(u[4] - u[3], 4.0 * (u[3] - u[2]));
@@ -100,7 +100,7 @@ __device__ double mp7(const double* u)
 }
 
 // MP5LD, src/flux.F90:556-633
-__device__ double mp5ld(const double* u, double w)
+__device__ __forceinline__ double mp5ld(const double* u, double w)
 {
     const double vadp = 1.666666666666667e-2 * w;
     const double ul = (-vadp + 3.333333333333333e-2) * u[0] + (5.0 * vadp - 2.166666666666667e-1) * u[1] +
@@ -112,7 +112,7 @@ __device__ double mp5ld(const double* u, double w)
 }
 
 // MP7LD, src/flux.F90:635-706: the limiter is switched by the shock flag
-__device__ double mp7ld(const double* u, double w, bool lskt)
+__device__ __forceinline__ double mp7ld(const double* u, double w, bool lskt)
 {
     const double vadp = 3.571428571428571e-3 * w;
     const double ul = (1.0 * vadp - 7.142857142857143e-3) * u[0] +
@@ -127,7 +127,7 @@ __device__ double mp7ld(const double* u, double w, bool lskt)
 }
 
 // WENO5 / WENO5Z, src/flux.F90:761-821,936-994
-__device__ double weno5(const double* u, bool z)
+__device__ __forceinline__ double weno5(const double* u, bool z)
 {
     const double uh0 = 0.333333333333333 * u[0] - 1.16666666666667 * u[1] + 1.83333333333333 * u[2];
     const double uh1 = -0.166666666666667 * u[1] + 0.833333333333333 * u[2] + 0.333333333333333 * u[3];
@@ -157,7 +157,7 @@ __device__ double weno5(const double* u, bool z)
 }
 
 // WENO7 / WENO7Z, src/flux.F90:826-925,999-1050
-__device__ double weno7(const double* u, bool z)
+__device__ __forceinline__ double weno7(const double* u, bool z)
 {
     double uh[4], bt[4];
     uh[0] = -0.25 * u[0] + 1.083333333333333 * u[1] - 1.916666666666667 * u[2] +
@@ -199,7 +199,7 @@ __device__ double weno7(const double* u, bool z)
 }
 
 // ROUND, src/flux.F90:717-752
-__device__ double round3(const double* u)
+__device__ __forceinline__ double round3(const double* u)
 {
     const double z0c = (u[1] - u[0] + 1.e-16) / (u[2] - u[0] + 1.e-16);
     const double a1c = 1.0 + 12.0 * z0c * z0c;
@@ -217,40 +217,33 @@ __device__ double round3(const double* u)
     return gc * (u[2] - u[0]) + u[0];
 }
 
-// recons_exp, src/flux.F90:269-350 (schemes checked at set-up).  LD false
-// leaves out the interior MP7-LD branch (reschem 5), whose registers would
-// otherwise set every scheme's occupancy: a caller with reschem 5 takes
-// LD true.
-template <bool LD = true>
-__device__ double recons_exp(const double* f, int inode, int dim, int ntype, int reschem,
-                             bool shock, double bfac)
+// recons_exp, src/flux.F90:269-350 (schemes checked at set-up).  The scheme
+// is a compile-time choice: with all of them in one kernel the one that needs
+// the most registers sets the occupancy of every other.
+template <int RS>
+__device__ __forceinline__ double recons_exp(const double* f, int inode, int dim, int ntype,
+                                             bool shock, double bfac)
 {
     if ((ntype == 1 && inode == 0) || (ntype == 2 && inode == dim - 1))
-        return reschem == -1 ? f[3] : 0.5 * (f[3] + f[4]);
+        return RS == -1 ? f[3] : 0.5 * (f[3] + f[4]);
     if ((ntype == 1 && inode == 1) || (ntype == 2 && inode == dim - 2))
-        return reschem == -1 ? f[3] : suw3(f + 2);
+        return RS == -1 ? f[3] : suw3(f + 2);
     if ((ntype == 1 && inode == 2) || (ntype == 2 && inode == dim - 3)) {
-        switch (reschem) {
-        case -1: return f[3];
-        case 0: return suw5(f + 1);
-        case 1: return weno5(f + 1, false);
-        case 2: return weno5(f + 1, true);
-        case 3: return mp5(f + 1);
-        case 5: return mp5ld(f + 1, bfac);
-        default: return round3(f + 2);
-        }
+        if constexpr (RS == -1) return f[3];
+        else if constexpr (RS == 0) return suw5(f + 1);
+        else if constexpr (RS == 1) return weno5(f + 1, false);
+        else if constexpr (RS == 2) return weno5(f + 1, true);
+        else if constexpr (RS == 3) return mp5(f + 1);
+        else if constexpr (RS == 5) return mp5ld(f + 1, bfac);
+        else return round3(f + 2);
     }
-    switch (reschem) {
-    case -1: return f[3];
-    case 0: return suw7(f);
-    case 1: return weno7(f, false);
-    case 2: return weno7(f, true);
-    case 3: return mp7(f);
-    case 5:
-        if constexpr (LD) return mp7ld(f, bfac, shock);
-        else return __builtin_nan("");  // not reached: reschem 5 runs with LD true
-    default: return round3(f + 2);
-    }
+    if constexpr (RS == -1) return f[3];
+    else if constexpr (RS == 0) return suw7(f);
+    else if constexpr (RS == 1) return weno7(f, false);
+    else if constexpr (RS == 2) return weno7(f, true);
+    else if constexpr (RS == 3) return mp7(f);
+    else if constexpr (RS == 5) return mp7ld(f, bfac, shock);
+    else return round3(f + 2);
 }
 
 // flux_steger_warming at one node, src/riemann.F90:23-161 (no species);
@@ -315,7 +308,7 @@ struct Roe {
     int br;  // which normal component carries the 3rd/4th eigenvectors
 };
 
-__device__ Roe roe_state(double gamma, double ro_l, double p_l, double e_l, const double* vel_l,
+__device__ __forceinline__ Roe roe_state(double gamma, double ro_l, double p_l, double e_l, const double* vel_l,
                          const double* ddi_l, double ro_r, double p_r, double e_r,
                          const double* vel_r, const double* ddi_r)
 {
@@ -348,113 +341,100 @@ __device__ Roe roe_state(double gamma, double ro_l, double p_l, double e_l, cons
     return r;
 }
 
-// row m (0..4) of LEV
+// row m (0..4) of LEV.  (The scalars are read, and the row written, in one
+// place: with m known only at run time the branches' accesses would
+// otherwise be merged through pointers, which puts both in scratch memory.)
 __device__ __forceinline__ void lev_row(const Roe& r, int m, double* l)
 {
-    switch (m) {
-    case 0:
-        l[0] = 0.5 * (r.b2 + r.ugp * r.rcs);
-        l[1] = -0.5 * (r.b1 * r.u1 + r.g1 * r.rcs);
-        l[2] = -0.5 * (r.b1 * r.u2 + r.g2 * r.rcs);
-        l[3] = -0.5 * (r.b1 * r.u3 + r.g3 * r.rcs);
-        l[4] = 0.5 * r.b1;
-        return;
-    case 1:
-        l[0] = 1.0 - r.b2;
-        l[1] = r.b1 * r.u1;
-        l[2] = r.b1 * r.u2;
-        l[3] = r.b1 * r.u3;
-        l[4] = -r.b1;
-        return;
-    case 4:
-        l[0] = 0.5 * (r.b2 - r.ugp * r.rcs);
-        l[1] = -0.5 * (r.b1 * r.u1 - r.g1 * r.rcs);
-        l[2] = -0.5 * (r.b1 * r.u2 - r.g2 * r.rcs);
-        l[3] = -0.5 * (r.b1 * r.u3 - r.g3 * r.rcs);
-        l[4] = 0.5 * r.b1;
-        return;
-    }
-    const double rgp = r.rgp;
-    l[4] = 0.0;
-    if (r.br == 0) {
-        if (m == 2) {
-            l[0] = (r.ugp * r.g2 - r.u2) * rgp;
-            l[1] = -r.g2;
-            l[2] = (1.0 - r.g2 * r.g2) * rgp;
-            l[3] = -r.g2 * r.g3 * rgp;
-        } else {
-            l[0] = (r.ugp * r.g3 - r.u3) * rgp;
-            l[1] = -r.g3;
-            l[2] = -r.g2 * r.g3 * rgp;
-            l[3] = (1.0 - r.g3 * r.g3) * rgp;
-        }
-    } else if (r.br == 1) {
-        if (m == 2) {
-            l[0] = (r.ugp * r.g1 - r.u1) * rgp;
-            l[1] = (1.0 - r.g1 * r.g1) * rgp;
-            l[2] = -r.g1;
-            l[3] = -r.g1 * r.g3 * rgp;
-        } else {
-            l[0] = (r.ugp * r.g3 - r.u3) * rgp;
-            l[1] = -r.g1 * r.g3 * rgp;
-            l[2] = -r.g3;
-            l[3] = (1.0 - r.g3 * r.g3) * rgp;
-        }
+    const double u1 = r.u1, u2 = r.u2, u3 = r.u3, rcs = r.rcs, g1 = r.g1, g2 = r.g2, g3 = r.g3;
+    const double ugp = r.ugp, b1 = r.b1, b2 = r.b2, rgp = r.rgp;
+    double l0, l1, l2, l3, l4;
+    if (m == 0) {
+        l0 = 0.5 * (b2 + ugp * rcs);
+        l1 = -0.5 * (b1 * u1 + g1 * rcs);
+        l2 = -0.5 * (b1 * u2 + g2 * rcs);
+        l3 = -0.5 * (b1 * u3 + g3 * rcs);
+        l4 = 0.5 * b1;
+    } else if (m == 1) {
+        l0 = 1.0 - b2;
+        l1 = b1 * u1;
+        l2 = b1 * u2;
+        l3 = b1 * u3;
+        l4 = -b1;
+    } else if (m == 4) {
+        l0 = 0.5 * (b2 - ugp * rcs);
+        l1 = -0.5 * (b1 * u1 - g1 * rcs);
+        l2 = -0.5 * (b1 * u2 - g2 * rcs);
+        l3 = -0.5 * (b1 * u3 - g3 * rcs);
+        l4 = 0.5 * b1;
     } else {
-        if (m == 2) {
-            l[0] = (r.ugp * r.g1 - r.u1) * rgp;
-            l[1] = (1.0 - r.g1 * r.g1) * rgp;
-            l[2] = -r.g1 * r.g2 * rgp;
-            l[3] = -r.g1;
-        } else {
-            l[0] = (r.ugp * r.g2 - r.u2) * rgp;
-            l[1] = -r.g1 * r.g2 * rgp;
-            l[2] = (1.0 - r.g2 * r.g2) * rgp;
-            l[3] = -r.g2;
-        }
+        // ga the component that carries the eigenvectors, gb and gc the
+        // others in order; row 2 belongs to gb, row 3 to gc
+        const bool two = m == 2;
+        const double gb = r.br == 0 ? g2 : g1, gc = r.br == 2 ? g2 : g3;
+        const double gm = two ? gb : gc;
+        const double um = two ? (r.br == 0 ? u2 : u1) : (r.br == 2 ? u2 : u3);
+        const double own = (1.0 - gm * gm) * rgp;
+        const double other = -gb * gc * rgp;
+        const double lb = two ? own : other, lc = two ? other : own;
+        l0 = (ugp * gm - um) * rgp;
+        l4 = 0.0;
+        l1 = r.br == 0 ? -gm : lb;
+        l2 = r.br == 1 ? -gm : (r.br == 0 ? lb : lc);
+        l3 = r.br == 2 ? -gm : lc;
     }
+    l[0] = l0;
+    l[1] = l1;
+    l[2] = l2;
+    l[3] = l3;
+    l[4] = l4;
 }
 
 // row m (0..4) of REV
 __device__ __forceinline__ void rev_row(const Roe& r, int m, double* v)
 {
-    const double c = r.cs;
-    switch (m) {
-    case 0:
-        v[0] = 1.0; v[1] = 1.0; v[2] = 0.0; v[3] = 0.0; v[4] = 1.0;
-        return;
-    case 4:
-        v[0] = r.hroe - r.ugp * c;
-        v[1] = r.hroe - 1.0 / r.b1;
-        v[4] = r.hroe + r.ugp * c;
+    const double c = r.cs, u1 = r.u1, u2 = r.u2, u3 = r.u3, g1 = r.g1, g2 = r.g2, g3 = r.g3;
+    const double hroe = r.hroe, ugp = r.ugp, b1 = r.b1;
+    double v0, v1, v2, v3, v4;
+    if (m == 0) {
+        v0 = 1.0; v1 = 1.0; v2 = 0.0; v3 = 0.0; v4 = 1.0;
+    } else if (m == 4) {
+        v0 = hroe - ugp * c;
+        v1 = hroe - 1.0 / b1;
+        v4 = hroe + ugp * c;
         if (r.br == 0) {
-            v[2] = r.u2 * r.g1 - r.u1 * r.g2;
-            v[3] = r.u3 * r.g1 - r.u1 * r.g3;
+            v2 = u2 * g1 - u1 * g2;
+            v3 = u3 * g1 - u1 * g3;
         } else if (r.br == 1) {
-            v[2] = r.u1 * r.g2 - r.u2 * r.g1;
-            v[3] = r.u3 * r.g2 - r.u2 * r.g3;
+            v2 = u1 * g2 - u2 * g1;
+            v3 = u3 * g2 - u2 * g3;
         } else {
-            v[2] = r.u1 * r.g3 - r.u3 * r.g1;
-            v[3] = r.u2 * r.g3 - r.u3 * r.g2;
+            v2 = u1 * g3 - u3 * g1;
+            v3 = u2 * g3 - u3 * g2;
         }
-        return;
-    }
-    const double um = m == 1 ? r.u1 : (m == 2 ? r.u2 : r.u3);
-    const double gm = m == 1 ? r.g1 : (m == 2 ? r.g2 : r.g3);
-    v[0] = um - c * gm;
-    v[1] = um;
-    v[4] = um + c * gm;
-    // columns 3 and 4 (src/solver.F90:2095-2146)
-    if (r.br == 0) {
-        v[2] = m == 1 ? -r.g2 : (m == 2 ? r.g1 : 0.0);
-        v[3] = m == 1 ? -r.g3 : (m == 2 ? 0.0 : r.g1);
-    } else if (r.br == 1) {
-        v[2] = m == 1 ? r.g2 : (m == 2 ? -r.g1 : 0.0);
-        v[3] = m == 1 ? 0.0 : (m == 2 ? -r.g3 : r.g2);
     } else {
-        v[2] = m == 1 ? r.g3 : (m == 2 ? 0.0 : -r.g1);
-        v[3] = m == 1 ? 0.0 : (m == 2 ? r.g3 : -r.g2);
+        const double um = m == 1 ? u1 : (m == 2 ? u2 : u3);
+        const double gm = m == 1 ? g1 : (m == 2 ? g2 : g3);
+        v0 = um - c * gm;
+        v1 = um;
+        v4 = um + c * gm;
+        // columns 3 and 4 (src/solver.F90:2095-2146)
+        if (r.br == 0) {
+            v2 = m == 1 ? -g2 : (m == 2 ? g1 : 0.0);
+            v3 = m == 1 ? -g3 : (m == 2 ? 0.0 : g1);
+        } else if (r.br == 1) {
+            v2 = m == 1 ? g2 : (m == 2 ? -g1 : 0.0);
+            v3 = m == 1 ? 0.0 : (m == 2 ? -g3 : g2);
+        } else {
+            v2 = m == 1 ? g3 : (m == 2 ? 0.0 : -g1);
+            v3 = m == 1 ? 0.0 : (m == 2 ? g3 : -g2);
+        }
     }
+    v[0] = v0;
+    v[1] = v1;
+    v[2] = v2;
+    v[3] = v3;
+    v[4] = v4;
 }
 
 }  // namespace uwd
