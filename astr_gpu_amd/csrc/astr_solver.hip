@@ -31,12 +31,15 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
+#include <condition_variable>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <type_traits>
 #include <vector>
 
@@ -4778,42 +4781,206 @@ int do_stats(astr_ctx* c, double* out)
     return ASTR_OK;
 }
 
-// host haloed Fortran array <-> device padded field
-int upload_field(astr_ctx* c, double* dev, const double* host, std::vector<double>& stage)
+// ---- host arrays <-> device fields
+//
+// Fields cross in chunks of the padded layout through pinned buffers: a
+// chunk's DMA (57 GB/s here) runs while another's rows are copied between
+// the buffer and the caller's array, and several threads do that copying,
+// which one thread does at 8 GB/s, page faults of a fresh array included.
+// (A pageable hipMemcpy of each padded field followed by one thread's row
+// copies moved 5-6 GB/s.)  The buffers belong to the process, as a transfer
+// needs them only while it runs: at most PIN_MAX of them, lent to one worker
+// of one call at a time, freed when the last context goes.
+
+constexpr size_t PIN_HALF = (size_t)2 << 20;  // bytes of a half: a worker fills one while
+                                              // the other's DMA runs
+constexpr int PIN_MAX = 16;                   // buffers of two halves: 64 MB in all
+constexpr int XFER_THREADS = 8;               // workers of one call
+
+struct PinPool {
+    std::mutex mu;
+    std::condition_variable cv;
+    std::vector<void*> idle;
+    int made = 0;      // buffers that exist, idle or lent
+    int contexts = 0;  // live contexts
+};
+PinPool& pin_pool()
 {
-    // work queued on the solver's stream may still read the field
-    HIPCHK(hipStreamSynchronize(c->stream));
-    const int ni = c->g.n[0] + 1 + 2 * HM, nj = c->g.n[1] + 1 + 2 * HM, nk = c->g.n[2] + 1 + 2 * HM;
-    stage.assign(c->nfield, 0.0);
-    for (int k = 0; k < nk; ++k)
-        for (int j = 0; j < nj; ++j)
-            memcpy(&stage[(OI - HM) + (long)j * c->pi + (long)k * c->pi * c->pj],
-                   host + (long)ni * (j + (long)nj * k), sizeof(double) * ni);
-    HIPCHK(hipMemcpy(dev, stage.data(), sizeof(double) * c->nfield, hipMemcpyHostToDevice));
+    static PinPool* p = new PinPool();  // (never destroyed: contexts may outlive static objects)
+    return *p;
+}
+
+// up to `want` buffers, at least one: waits while every buffer is lent
+// (their holders wait for nobody).  Empty where pinned memory is refused.
+std::vector<void*> pin_take(int want)
+{
+    PinPool& P = pin_pool();
+    std::vector<void*> got;
+    std::unique_lock<std::mutex> lk(P.mu);
+    P.cv.wait(lk, [&] { return !P.idle.empty() || P.made < PIN_MAX; });
+    while ((int)got.size() < want && !P.idle.empty()) {
+        got.push_back(P.idle.back());
+        P.idle.pop_back();
+    }
+    while ((int)got.size() < want && P.made < PIN_MAX) {
+        void* b = nullptr;
+        if (hipHostMalloc(&b, 2 * PIN_HALF, hipHostMallocPortable) != hipSuccess) {
+            (void)hipGetLastError();
+            break;
+        }
+        ++P.made;
+        got.push_back(b);
+    }
+    return got;
+}
+
+void pin_give(std::vector<void*>& bufs)
+{
+    PinPool& P = pin_pool();
+    {
+        std::lock_guard<std::mutex> lk(P.mu);
+        P.idle.insert(P.idle.end(), bufs.begin(), bufs.end());
+    }
+    bufs.clear();
+    P.cv.notify_all();
+}
+
+void pin_context(int add)
+{
+    PinPool& P = pin_pool();
+    std::lock_guard<std::mutex> lk(P.mu);
+    P.contexts += add;
+    if (P.contexts > 0) return;
+    for (void* b : P.idle) (void)hipHostFree(b);
+    P.made -= (int)P.idle.size();
+    P.idle.clear();
+}
+
+// one field of a transfer: host is the haloed Fortran array, or that of the
+// nodes 0..n alone (interior)
+struct HostField {
+    double* dev;
+    double* host;
+    bool interior;
+};
+
+// the chunk [e0, e1) of a padded field, elements in the device layout: its
+// rows' host parts copied to (up) or from the buffer, the rows' padding
+// zero on the way up
+void copy_chunk(const astr_ctx* c, const HostField& f, double* buf, long e0, long e1, bool up)
+{
+    const long off = f.interior ? OI : OI - HM;
+    const long len = c->g.n[0] + 1 + (f.interior ? 0 : 2 * HM);
+    const long nj = c->g.n[1] + 1, nk = c->g.n[2] + 1;
+    for (long r = e0 / c->pi; r * c->pi < e1; ++r) {
+        long hr = r;
+        if (f.interior) {
+            const long j = r % c->pj - HM, k = r / c->pj - HM;
+            if (j < 0 || j >= nj || k < 0 || k >= nk) continue;
+            hr = j + nj * k;
+        }
+        const long r0 = r * c->pi;
+        const long lo = std::max(e0, r0 + off), hi = std::min(e1, r0 + off + len);
+        double* h = f.host + hr * len;  // the row's host part, from element r0 + off
+        if (!up) {
+            if (lo < hi) memcpy(h + (lo - r0 - off), buf + (lo - e0), sizeof(double) * (hi - lo));
+            continue;
+        }
+        for (long e = std::max(e0, r0); e < std::min(e1, r0 + off); ++e) buf[e - e0] = 0.0;
+        if (lo < hi) memcpy(buf + (lo - e0), h + (lo - r0 - off), sizeof(double) * (hi - lo));
+        for (long e = std::max(e0, r0 + off + len); e < std::min(e1, r0 + c->pi); ++e)
+            buf[e - e0] = 0.0;
+    }
+}
+
+// every field up to, or down from, the device, in order with the context's
+// stream; returns when the host arrays are read or written
+int transfer(astr_ctx* c, const std::vector<HostField>& fields, bool up)
+{
+    const long total = c->nfield * (long)fields.size();
+    const size_t bytes = sizeof(double) * (size_t)total;
+    // a worker for every 2 MB: below that its start costs more than it gives
+    const int want = (int)std::min<size_t>(XFER_THREADS, 1 + bytes / PIN_HALF);
+    std::vector<void*> bufs = pin_take(want);
+    if (bufs.empty()) return fail(ASTR_E_NOMEM, "pinned host buffer");
+    const int nw = (int)bufs.size();
+    // chunks of at most a half, and a few for each worker's two halves
+    const long chunk = std::max<long>(
+        std::min<long>((long)(PIN_HALF / sizeof(double)), (total / nw + 3) / 4), 8192);
+    const long per = (c->nfield + chunk - 1) / chunk, nchunks = per * (long)fields.size();
+    std::atomic<long> next{0};
+    std::atomic<int> err{(int)hipSuccess};
+    auto work = [&](double* buf) {
+        double* half[2] = {buf, buf + PIN_HALF / sizeof(double)};
+        hipEvent_t ev[2] = {nullptr, nullptr};
+        long at[2] = {-1, -1};  // the chunk whose DMA is in a half
+        auto ok = [&](hipError_t e) {
+            if (e != hipSuccess) err = (int)e;
+            return e == hipSuccess;
+        };
+        auto finish = [&](int h) {  // the DMA of half h, and the rows on the way down
+            if (at[h] < 0) return;
+            const long k = at[h];
+            at[h] = -1;
+            if (!ok(hipEventSynchronize(ev[h])) || up) return;
+            const long e0 = (k % per) * chunk;
+            copy_chunk(c, fields[k / per], half[h], e0, std::min(e0 + chunk, c->nfield), false);
+        };
+        if (ok(hipSetDevice(c->device)) &&
+            ok(hipEventCreateWithFlags(&ev[0], hipEventDisableTiming)) &&
+            ok(hipEventCreateWithFlags(&ev[1], hipEventDisableTiming))) {
+            int h = 0;
+            while (err == (int)hipSuccess) {
+                finish(h);
+                const long k = next++;
+                if (k >= nchunks) break;
+                const HostField& f = fields[k / per];
+                const long e0 = (k % per) * chunk, e1 = std::min(e0 + chunk, c->nfield);
+                const size_t nb = sizeof(double) * (size_t)(e1 - e0);
+                if (up) {
+                    copy_chunk(c, f, half[h], e0, e1, true);
+                    if (!ok(hipMemcpyAsync(f.dev + e0, half[h], nb, hipMemcpyHostToDevice, c->stream)))
+                        break;
+                } else if (!ok(hipMemcpyAsync(half[h], f.dev + e0, nb, hipMemcpyDeviceToHost,
+                                              c->stream))) {
+                    break;
+                }
+                at[h] = k;
+                if (!ok(hipEventRecord(ev[h], c->stream))) {
+                    (void)hipStreamSynchronize(c->stream);
+                    at[h] = -1;
+                    break;
+                }
+                h ^= 1;
+            }
+            finish(0);
+            finish(1);
+        }
+        for (int h = 0; h < 2; ++h)
+            if (ev[h]) (void)hipEventDestroy(ev[h]);
+    };
+    std::vector<std::thread> ts;
+    try {
+        for (int w = 1; w < nw; ++w) ts.emplace_back(work, (double*)bufs[w]);
+    } catch (...) {
+        // no more threads: the ones that started, and this one, do the work
+    }
+    work((double*)bufs[0]);
+    for (std::thread& t : ts) t.join();
+    pin_give(bufs);
+    if (err != (int)hipSuccess)
+        return fail(ASTR_E_HIP, std::string("host transfer: ") + hipGetErrorString((hipError_t)err.load()));
     return ASTR_OK;
 }
 
-int download_field(astr_ctx* c, const double* dev, double* host, std::vector<double>& stage,
-                   bool interior)
+int upload_field(astr_ctx* c, double* dev, const double* host)
 {
-    stage.resize(c->nfield);
-    HIPCHK(hipMemcpy(stage.data(), dev, sizeof(double) * c->nfield, hipMemcpyDeviceToHost));
-    if (interior) {
-        const int ni = c->g.n[0] + 1, nj = c->g.n[1] + 1, nk = c->g.n[2] + 1;
-        for (int k = 0; k < nk; ++k)
-            for (int j = 0; j < nj; ++j)
-                memcpy(host + (long)ni * (j + (long)nj * k),
-                       &stage[c->g.org + (long)j * c->pi + (long)k * c->pi * c->pj],
-                       sizeof(double) * ni);
-    } else {
-        const int ni = c->g.n[0] + 1 + 2 * HM, nj = c->g.n[1] + 1 + 2 * HM, nk = c->g.n[2] + 1 + 2 * HM;
-        for (int k = 0; k < nk; ++k)
-            for (int j = 0; j < nj; ++j)
-                memcpy(host + (long)ni * (j + (long)nj * k),
-                       &stage[(OI - HM) + (long)j * c->pi + (long)k * c->pi * c->pj],
-                       sizeof(double) * ni);
-    }
-    return ASTR_OK;
+    return transfer(c, {{dev, const_cast<double*>(host), false}}, true);
+}
+
+int download_field(astr_ctx* c, const double* dev, double* host, bool interior)
+{
+    return transfer(c, {{const_cast<double*>(dev), host, interior}}, false);
 }
 
 int time_mark(astr_ctx* c, int slot)
@@ -5670,6 +5837,7 @@ int astr_create(const astr_params* p, int32_t device, astr_ctx** out)
                         "the line sweeps' LDS tiles exceed the device's limit per workgroup");
     }
     auto* c = new astr_ctx();
+    pin_context(1);
     c->p = *p;
     c->device = device;
     for (int d = 0; d < 3; ++d) c->lines_ok[d] = lines_ok[d];
@@ -5860,6 +6028,7 @@ int astr_destroy(astr_ctx* c)
         if (c->ev[e]) (void)hipEventDestroy(c->ev[e]);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
+    pin_context(-1);
     return ASTR_OK;
 }
 
@@ -5895,7 +6064,6 @@ int astr_upload_geom(astr_ctx* c, const double* jacob, const double* dxi)
                         else if (slot != v) { rect = false; break; }
                     }
         }
-    std::vector<double> stage;
     if (rect) {
         HIPCHK(hipMemcpy(c->xi, xi.data(), sizeof(double) * xi.size(), hipMemcpyHostToDevice));
         c->curv = false;
@@ -5915,10 +6083,10 @@ int astr_upload_geom(astr_ctx* c, const double* jacob, const double* dxi)
         }
         for (int d = 0; d < 3; ++d)
             for (int e = 0; e < 3; ++e)
-                TRY(upload_field(c, c->dxf[3 * d + e], dxi + (long)(d + 3 * e) * nt, stage));
+                TRY(upload_field(c, c->dxf[3 * d + e], dxi + (long)(d + 3 * e) * nt));
         c->curv = true;
     }
-    TRY(upload_field(c, c->jac, jacob, stage));
+    TRY(upload_field(c, c->jac, jacob));
     // a uniform grid's jacob is one value: the kernels of the central path
     // then take it as a scalar (the array stays uploaded for the others)
     c->juni = true;
@@ -5934,12 +6102,14 @@ int astr_upload_state(astr_ctx* c, const double* q, const double* rho, const dou
     if (!c || !q || !rho || !vel || !prs || !tmp) return fail(ASTR_E_ARG, "null argument");
     TRY(set_dev(c));
     const long nt = (long)(c->g.n[0] + 1 + 2 * HM) * (c->g.n[1] + 1 + 2 * HM) * (c->g.n[2] + 1 + 2 * HM);
-    std::vector<double> stage;
-    for (int m = 0; m < 5; ++m) TRY(upload_field(c, c->q[m], q + m * nt, stage));
-    TRY(upload_field(c, c->prim[0], rho, stage));
-    for (int m = 0; m < 3; ++m) TRY(upload_field(c, c->prim[1 + m], vel + m * nt, stage));
-    TRY(upload_field(c, c->prim[4], prs, stage));
-    TRY(upload_field(c, c->prim[5], tmp, stage));
+    std::vector<HostField> fs;
+    auto add = [&](double* dev, const double* h) { fs.push_back({dev, const_cast<double*>(h), false}); };
+    for (int m = 0; m < 5; ++m) add(c->q[m], q + m * nt);
+    add(c->prim[0], rho);
+    for (int m = 0; m < 3; ++m) add(c->prim[1 + m], vel + m * nt);
+    add(c->prim[4], prs);
+    add(c->prim[5], tmp);
+    TRY(transfer(c, fs, true));
     c->have_state = true;
     return ASTR_OK;
 }
@@ -5948,34 +6118,32 @@ int astr_download_state(astr_ctx* c, double* q, double* rho, double* vel, double
 {
     if (!c || !q || !rho || !vel || !prs || !tmp) return fail(ASTR_E_ARG, "null argument");
     TRY(set_dev(c));
-    HIPCHK(hipStreamSynchronize(c->stream));
     const long nt = (long)(c->g.n[0] + 1 + 2 * HM) * (c->g.n[1] + 1 + 2 * HM) * (c->g.n[2] + 1 + 2 * HM);
-    std::vector<double> stage;
-    for (int m = 0; m < 5; ++m) TRY(download_field(c, c->q[m], q + m * nt, stage, false));
-    TRY(download_field(c, c->prim[0], rho, stage, false));
-    for (int m = 0; m < 3; ++m) TRY(download_field(c, c->prim[1 + m], vel + m * nt, stage, false));
-    TRY(download_field(c, c->prim[4], prs, stage, false));
-    TRY(download_field(c, c->prim[5], tmp, stage, false));
-    return ASTR_OK;
+    std::vector<HostField> fs;
+    for (int m = 0; m < 5; ++m) fs.push_back({c->q[m], q + m * nt, false});
+    fs.push_back({c->prim[0], rho, false});
+    for (int m = 0; m < 3; ++m) fs.push_back({c->prim[1 + m], vel + m * nt, false});
+    fs.push_back({c->prim[4], prs, false});
+    fs.push_back({c->prim[5], tmp, false});
+    return transfer(c, fs, false);
 }
 
 int astr_download_rhs(astr_ctx* c, double* qrhs, double* dvel, double* dtmp)
 {
     if (!c) return fail(ASTR_E_ARG, "null argument");
     TRY(set_dev(c));
-    HIPCHK(hipStreamSynchronize(c->stream));
     const long ni = n_interior(c);
-    std::vector<double> stage;
+    std::vector<HostField> fs;
     if (qrhs)
-        for (int m = 0; m < 5; ++m) TRY(download_field(c, c->qrhs[m], qrhs + m * ni, stage, true));
+        for (int m = 0; m < 5; ++m) fs.push_back({c->qrhs[m], qrhs + m * ni, true});
     if (dvel)
         for (int m = 0; m < 3; ++m)
             for (int d = 0; d < 3; ++d)
                 // dvel(:,:,:,m,d) is column (m-1) + 3*(d-1) of the Fortran array
-                TRY(download_field(c, c->dvel[m * 3 + d], dvel + (m + 3 * d) * ni, stage, true));
+                fs.push_back({c->dvel[m * 3 + d], dvel + (m + 3 * d) * ni, true});
     if (dtmp)
-        for (int d = 0; d < 3; ++d) TRY(download_field(c, c->dtmp[d], dtmp + d * ni, stage, true));
-    return ASTR_OK;
+        for (int d = 0; d < 3; ++d) fs.push_back({c->dtmp[d], dtmp + d * ni, true});
+    return fs.empty() ? ASTR_OK : transfer(c, fs, false);
 }
 
 static int ready_state(astr_ctx* c)
@@ -6704,8 +6872,7 @@ static int field_op(astr_ctx* c, int dir, const double* f, double* df, int pass)
     if (!c || !f || !df) return fail(ASTR_E_ARG, "null argument");
     if (dir < 1 || dir > ndims_of(c)) return fail(ASTR_E_ARG, "dir must be 1..3 (1..2 in 2-D)");
     TRY(set_dev(c));
-    std::vector<double> stage;
-    TRY(upload_field(c, c->scratch, f, stage));
+    TRY(upload_field(c, c->scratch, f));
     if (pass == PASS_DERIV_FIELD && c->p.deriv_explicit) {
         FieldXArgs a{};
         a.g = c->g;
@@ -6723,9 +6890,7 @@ static int field_op(astr_ctx* c, int dir, const double* f, double* df, int pass)
         a.fout = c->scratch2;
         TRY(launch_sweep(c, a));
     }
-    HIPCHK(hipStreamSynchronize(c->stream));
-    TRY(download_field(c, c->scratch2, df, stage, true));
-    return ASTR_OK;
+    return download_field(c, c->scratch2, df, true);
 }
 
 int astr_deriv_field(astr_ctx* c, int32_t dir, const double* f, double* df)
@@ -6749,8 +6914,7 @@ int astr_flux_field(astr_ctx* c, int32_t dir, int32_t wind, int32_t shock, const
     TRY(set_dev(c));
     const int d = dir - 1;
     const int nts[3] = {c->p.npdci, c->p.npdcj, c->p.npdck};
-    std::vector<double> stage;
-    TRY(upload_field(c, c->scratch, f, stage));
+    TRY(upload_field(c, c->scratch, f));
     HIPCHK(hipMemsetAsync(c->scratch2, 0, sizeof(double) * c->nfield, c->stream));
     const int da = d == 0 ? 1 : 0, db = d == 2 ? 1 : 2;
     if (c->p.convection == 2) {
@@ -6796,9 +6960,7 @@ int astr_flux_field(astr_ctx* c, int32_t dir, int32_t wind, int32_t shock, const
                            c->stream, ra);
     }
     HIPCHK(hipGetLastError());
-    HIPCHK(hipStreamSynchronize(c->stream));
-    TRY(download_field(c, c->scratch2, fh, stage, false));
-    return ASTR_OK;
+    return download_field(c, c->scratch2, fh, false);
 }
 
 int astr_adjoint_record(astr_ctx* c, int32_t nsteps, double dt, int32_t ckpt, double* J)
@@ -6888,16 +7050,11 @@ int astr_adjoint_reverse(astr_ctx* c, double* qbar, double* pbar, double* ms)
     }
     // the adjoint of the initial state, haloed host layout
     const AdjFields f = adj_fields(c);
-    std::vector<double> stage, one((size_t)n_haloed(c));
     const long nh = n_haloed(c);
-    for (int m = 0; m < 5; ++m) {
-        TRY(download_field(c, f.qb[m], one.data(), stage, false));
-        memcpy(qbar + m * nh, one.data(), sizeof(double) * nh);
-    }
-    for (int m = 0; m < 6; ++m) {
-        TRY(download_field(c, f.pb[m], one.data(), stage, false));
-        memcpy(pbar + m * nh, one.data(), sizeof(double) * nh);
-    }
+    std::vector<HostField> fs;
+    for (int m = 0; m < 5; ++m) fs.push_back({f.qb[m], qbar + m * nh, false});
+    for (int m = 0; m < 6; ++m) fs.push_back({f.pb[m], pbar + m * nh, false});
+    TRY(transfer(c, fs, false));
     // leave the device state at the end of the forward steps, as the
     // record left it (after the objective's qswap and gradients)
     TRY(load_state(c, nseg));
@@ -6936,15 +7093,13 @@ int astr_line_adjoint(astr_ctx* c, int32_t op, int32_t dir, int32_t wrap, const 
     if (op == 0 && c->p.deriv_explicit)
         return fail(ASTR_E_UNSUPPORTED, "the transposed derivative is the compact one");
     TRY(set_dev(c));
-    std::vector<double> stage;
-    TRY(upload_field(c, c->scratch, gbar, stage));
+    TRY(upload_field(c, c->scratch, gbar));
     HIPCHK(hipMemsetAsync(c->scratch2, 0, sizeof(double) * c->nfield, c->stream));
     const double* fin[1] = {c->scratch};
     double* fout[1] = {c->scratch2};
     TRY(launch_sweep_t(c, dir - 1, op == 0 ? OP_DERIV : OP_FILTER, 1, fin, fout, nullptr, wrap != 0,
                        false));
-    HIPCHK(hipStreamSynchronize(c->stream));
-    return download_field(c, c->scratch2, fbar, stage, false);
+    return download_field(c, c->scratch2, fbar, false);
 }
 
 }  // extern "C"

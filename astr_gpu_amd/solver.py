@@ -82,9 +82,9 @@ class AstrSolver:
 
     def download_state(self) -> dict:
         s = haloed_shape(self.p)
-        out = {"q": np.zeros(s + (5,), order="F"), "rho": np.zeros(s, order="F"),
-               "vel": np.zeros(s + (3,), order="F"), "prs": np.zeros(s, order="F"),
-               "tmp": np.zeros(s, order="F")}
+        out = {"q": np.empty(s + (5,), order="F"), "rho": np.empty(s, order="F"),
+               "vel": np.empty(s + (3,), order="F"), "prs": np.empty(s, order="F"),
+               "tmp": np.empty(s, order="F")}
         check(self.lib.astr_download_state(self.ctx, dptr(out["q"]), dptr(out["rho"]),
                                            dptr(out["vel"]), dptr(out["prs"]),
                                            dptr(out["tmp"])), "astr_download_state")
@@ -92,8 +92,8 @@ class AstrSolver:
 
     def download_rhs(self) -> dict:
         s = (self.p.im + 1, self.p.jm + 1, self.p.km + 1)
-        out = {"qrhs": np.zeros(s + (5,), order="F"), "dvel": np.zeros(s + (3, 3), order="F"),
-               "dtmp": np.zeros(s + (3,), order="F")}
+        out = {"qrhs": np.empty(s + (5,), order="F"), "dvel": np.empty(s + (3, 3), order="F"),
+               "dtmp": np.empty(s + (3,), order="F")}
         check(self.lib.astr_download_rhs(self.ctx, dptr(out["qrhs"]), dptr(out["dvel"]),
                                          dptr(out["dtmp"])), "astr_download_rhs")
         return out
@@ -151,7 +151,7 @@ class AstrSolver:
         along direction (1..3) applied to gbar (haloed; nodes 0..n used):
         the haloed adjoint of the operator's input (astr_line_adjoint)."""
         g = self._f(gbar, haloed_shape(self.p))
-        out = np.zeros(haloed_shape(self.p), order="F")
+        out = np.empty(haloed_shape(self.p), order="F")
         check(self.lib.astr_line_adjoint(self.ctx, int(op), int(direction), int(bool(wrap)),
                                          dptr(g), dptr(out)), "astr_line_adjoint")
         return out
@@ -161,8 +161,8 @@ class AstrSolver:
         current state and its gradient with respect to that state
         (astr_adjoint_enstrophy); ms = (forward, reversal) milliseconds."""
         J = np.zeros(1)
-        qb = np.zeros(haloed_shape(self.p, (5,)), order="F")
-        pb = np.zeros(haloed_shape(self.p, (6,)), order="F")
+        qb = np.empty(haloed_shape(self.p, (5,)), order="F")
+        pb = np.empty(haloed_shape(self.p, (6,)), order="F")
         ms = np.zeros(2)
         check(self.lib.astr_adjoint_enstrophy(self.ctx, int(nsteps), float(dt), int(ckpt),
                                               dptr(J), dptr(qb), dptr(pb), dptr(ms)),
@@ -183,8 +183,8 @@ class AstrSolver:
         """(qbar, pbar, ms): the gradient of the recorded J with respect to
         the recorded initial state, and the milliseconds of the reversal
         (astr_adjoint_reverse)."""
-        qb = np.zeros(haloed_shape(self.p, (5,)), order="F")
-        pb = np.zeros(haloed_shape(self.p, (6,)), order="F")
+        qb = np.empty(haloed_shape(self.p, (5,)), order="F")
+        pb = np.empty(haloed_shape(self.p, (6,)), order="F")
         ms = np.zeros(1)
         check(self.lib.astr_adjoint_reverse(self.ctx, dptr(qb), dptr(pb), dptr(ms)),
               "astr_adjoint_reverse")
@@ -259,7 +259,7 @@ class AstrSolver:
     def central(self, direction: int, f) -> np.ndarray:
         """fds%central along `direction` (1..3) for every line of field f."""
         f = self._f(f, haloed_shape(self.p))
-        df = np.zeros((self.p.im + 1, self.p.jm + 1, self.p.km + 1), order="F")
+        df = np.empty((self.p.im + 1, self.p.jm + 1, self.p.km + 1), order="F")
         check(self.lib.astr_deriv_field(self.ctx, int(direction), dptr(f), dptr(df)),
               "astr_deriv_field")
         return df
@@ -267,7 +267,7 @@ class AstrSolver:
     def compact_filter(self, direction: int, f) -> np.ndarray:
         """compact_filter along `direction` (1..3) for every line of field f."""
         f = self._f(f, haloed_shape(self.p))
-        ff = np.zeros((self.p.im + 1, self.p.jm + 1, self.p.km + 1), order="F")
+        ff = np.empty((self.p.im + 1, self.p.jm + 1, self.p.km + 1), order="F")
         check(self.lib.astr_filter_field(self.ctx, int(direction), dptr(f), dptr(ff)),
               "astr_filter_field")
         return ff
@@ -278,7 +278,7 @@ class AstrSolver:
         line; haloed result, entry i the interface i+1/2 (zero where no
         interface is computed)."""
         f = self._f(f, haloed_shape(self.p))
-        fh = np.zeros(haloed_shape(self.p), order="F")
+        fh = np.empty(haloed_shape(self.p), order="F")
         check(self.lib.astr_flux_field(self.ctx, int(direction), int(wind), int(bool(shock)),
                                        dptr(f), dptr(fh)), "astr_flux_field")
         return fh
