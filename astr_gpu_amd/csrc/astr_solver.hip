@@ -2500,7 +2500,8 @@ struct SensorArgs {
     const double* prs;
     double* ssf;
     unsigned char* lshock;
-    // k_grad_ssf: the velocity and the metric lines
+    unsigned lp, rb, nch, njb;  // sensor_pair's layout
+    // k_ssf of the velocity and the metric lines
     const double* vel[3];
     const double* xi[3];
     // a two-dimensional step: the pressure of the planes k = -1 and 1 is
@@ -2517,104 +2518,60 @@ struct SensorArgs {
 __host__ __device__ __forceinline__ bool lo_end(int nt) { return nt == 1 || nt == 4; }
 __host__ __device__ __forceinline__ bool hi_end(int nt) { return nt == 2 || nt == 4; }
 
-// ducrossensor, part 1 (src/commcal.F90:236-272), at one node from its
-// velocity gradients dv (3(m-1)+(n-1): dvel(m,n)); the pressure stencil is
-// clamped at a bounded end (ntype 1 and 2 in the reference, both ends of
-// ntype 4)
-__device__ __forceinline__ double ssf_of(const SensorArgs& a, int i, int j, int k, long gi,
-                                         const double* dv)
+// The nodes of the sensor's kernels: a thread takes two neighbours of a row
+// (i even), lp threads a piece of a row, and a workgroup the same piece of rb
+// rows; consecutive pieces go to one XCD, so that a row's neighbours come from
+// its L1 and L2.  The stencils are read two nodes to a load: one load takes
+// the address unit 16 cycles whatever its width, and these loads were what
+// bound the kernels (the unit was busy for four fifths of their time with
+// one node to a load).
+__device__ __forceinline__ bool sensor_pair(const SensorArgs& a, int& i, int& j, int& k)
 {
-    const double div = dv[0] + dv[4] + dv[8];
-    const double div2 = div * div;
-    const double vx = dv[7] - dv[5];  // dvel(3,2) - dvel(2,3)
-    const double vy = dv[2] - dv[6];  // dvel(1,3) - dvel(3,1)
-    const double vz = dv[3] - dv[1];  // dvel(2,1) - dvel(1,2)
-    const double vort = vx * vx + vy * vy + vz * vz;
-    int ip1 = i + 1, im1 = i - 1, jp1 = j + 1, jm1 = j - 1, kp1 = k + 1, km1 = k - 1;
-    if (lo_end(a.ntype[0]) && im1 < 0) im1 = 0;
-    if (lo_end(a.ntype[1]) && jm1 < 0) jm1 = 0;
-    if (lo_end(a.ntype[2]) && km1 < 0) km1 = 0;
-    if (hi_end(a.ntype[0]) && ip1 > a.g.n[0]) ip1 = a.g.n[0];
-    if (hi_end(a.ntype[1]) && jp1 > a.g.n[1]) jp1 = a.g.n[1];
-    if (hi_end(a.ntype[2]) && kp1 > a.g.n[2]) kp1 = a.g.n[2];
-    const double pc = a.prs[gi];
-    const double* P = a.prs;
-    const double pi1 = P[gidx(a.g, ip1, j, k)], pi0 = P[gidx(a.g, im1, j, k)];
-    const double pj1 = P[gidx(a.g, i, jp1, k)], pj0 = P[gidx(a.g, i, jm1, k)];
-    const double pk1 = a.p2d ? pc : P[gidx(a.g, i, j, kp1)];
-    const double pk0 = a.p2d ? pc : P[gidx(a.g, i, j, km1)];
-    const double dpdi = fabs(pi1 - 2.0 * pc + pi0) / (pi1 + 2.0 * pc + pi0);
-    const double dpdj = fabs(pj1 - 2.0 * pc + pj0) / (pj1 + 2.0 * pc + pj0);
-    const double dpdk = fabs(pk1 - 2.0 * pc + pk0) / (pk1 + 2.0 * pc + pk0);
-    return div2 / (div2 + vort + 1.e-30) * uwd::max2(uwd::max2(dpdi, dpdj), dpdk);
+    const unsigned per = gridDim.x / 8;
+    const unsigned w = (blockIdx.x & 7) * per + blockIdx.x / 8;  // the XCD's own run
+    const unsigned r = w / a.nch;
+    k = (int)(r / a.njb);
+    const unsigned jb = r - (unsigned)k * a.njb, tr = threadIdx.x / a.lp;
+    j = (int)(jb * a.rb + tr);
+    i = 2 * (int)((w - r * a.nch) * a.lp + threadIdx.x - tr * a.lp);
+    return tr < a.rb && k <= a.g.n[2] && j <= a.g.n[1] && i <= a.g.n[0];
+}
+unsigned sensor_layout(SensorArgs& a)
+{
+    const unsigned pairs = (unsigned)a.g.n[0] / 2 + 1;
+    a.nch = (pairs + 63) / 64;
+    a.lp = ((pairs + a.nch - 1) / a.nch + 7) / 8 * 8;
+    a.rb = 256 / a.lp;
+    a.njb = ((unsigned)a.g.n[1] + a.rb) / a.rb;
+    const long nb = (long)a.nch * a.njb * (a.g.n[2] + 1);
+    return (unsigned)((nb + 7) / 8 * 8);
 }
 
-__global__ void k_ducros_ssf(SensorArgs a)
+// two doubles through a 32-bit byte offset, as ldc
+typedef double d2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ d2 ldc2(const double* base, unsigned int boff)
 {
-    const long p = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long ni = a.g.n[0] + 1, nj = a.g.n[1] + 1;
-    if (p >= ni * nj * (a.g.n[2] + 1)) return;
-    int i, j, k;
-    split3(p, ni, nj, i, j, k);
-    const long gi = gidx(a.g, i, j, k);
-    double dv[9];
-#pragma unroll
-    for (int m = 0; m < 9; ++m) dv[m] = a.dvel[m][gi];
-    a.ssf[gi] = ssf_of(a, i, j, k, gi, dv);
+    return *(__attribute__((address_space(1))) const d2*)((gcptr)base + boff);
 }
 
-// ducrossensor, part 2 (src/commcal.F90:278-316): lshock = max of ssf over
-// offsets -hm+1..hm along each axis > shkcrt, clamped at bounded ends;
-// along a periodic axis the offsets wrap (dataswap(ssf), src/commcal.F90:
-// 276, src/parallel.F90:4170-4175, which a two-dimensional box's k axis does
-// not need: its planes repeat the plane itself).
-// A node whose windows leave no end of the box, all but a frame of them,
-// reads them at fixed distances: with the clamp and the 64-bit index of
-// every offset the kernel was bound by its index arithmetic (555 vector
-// instructions a wavefront).
-__global__ void k_ducros_flag(SensorArgs a)
+// diff6ec at node t of a line v(-hm..dim+hm), src/derivative.F90:350-413,
+// from v(t-3..t+3): no node's stencil leaves them
+__device__ __forceinline__ double diff6ec_w(const double (&w)[7], int t, int dim, int ntype)
 {
-    const long p = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long ni = a.g.n[0] + 1, nj = a.g.n[1] + 1;
-    if (p >= ni * nj * (a.g.n[2] + 1)) return;
-    int c0[3];
-    split3(p, ni, nj, c0[0], c0[1], c0[2]);
-    const long gi = gidx(a.g, c0[0], c0[1], c0[2]);
-    double m = 0.0;
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        if (d >= a.ndims) break;
-        const int n = a.g.n[d];
-        const double* f = a.ssf + gi;
-        if (c0[d] >= HM - 1 && c0[d] + HM <= n) {
-            const int sd = (int)a.g.s[d];
-#pragma unroll
-            for (int o = -HM + 1; o <= HM; ++o) m = uwd::max2(m, f[o * sd]);
-        } else {
-            for (int o = -HM + 1; o <= HM; ++o) {
-                int t = c0[d] + o;
-                if (a.ntype[d] == 3) t = t < 0 ? t + n : (t > n ? t - n : t);
-                if (lo_end(a.ntype[d]) && t < 0) t = 0;
-                if (hi_end(a.ntype[d]) && t > n) t = n;
-                // (a rank's interface end, ntype 1's high and 2's low: the
-                // halo, which no neighbour fills on one domain, is zero)
-                m = uwd::max2(m, t < 0 || t > n ? 0.0 : f[(long)(t - c0[d]) * a.g.s[d]]);
-            }
-        }
+    const bool lob = ntype == 1 || ntype == 4, hib = ntype == 2 || ntype == 4;
+    double r = 0.75 * (w[4] - w[2]) - 0.15 * (w[5] - w[1]) + (1.0 / 60.0) * (w[6] - w[0]);
+    if (lob && t <= 2) {
+        if (t == 0) r = -0.5 * w[5] + 2.0 * w[4] - 1.5 * w[3];
+        else if (t == 1) r = 0.5 * (w[4] - w[2]);
+        else r = (2.0 / 3.0) * (w[4] - w[2]) - (1.0 / 12.0) * (w[5] - w[1]);
+    } else if (hib && t >= dim - 2) {
+        if (t == dim) r = 0.5 * w[1] - 2.0 * w[2] + 1.5 * w[3];
+        else if (t == dim - 1) r = 0.5 * (w[4] - w[2]);
+        else r = (2.0 / 3.0) * (w[4] - w[2]) - (1.0 / 12.0) * (w[5] - w[1]);
     }
-    a.lshock[gi] = m > a.shkcrt ? 1 : 0;
+    return r;
 }
-
-struct GradXArgs {
-    Geo g;
-    int ntype[3], ndims;
-    const double* prim[6];
-    const double* xi[3];
-    double* dvel[9];
-    double* dtmp[3];
-};
-
-// diff6ec at node t of a line v(-hm..dim+hm), src/derivative.F90:350-413
+// The same from memory, which is read within the line's nodes at its ends
 __device__ __forceinline__ double diff6ec_at(const double* base, long stride, int t, int dim,
                                              int ntype)
 {
@@ -2630,6 +2587,178 @@ __device__ __forceinline__ double diff6ec_at(const double* base, long stride, in
     return 0.75 * (V(t + 1) - V(t - 1)) - 0.15 * (V(t + 2) - V(t - 2)) +
            (1.0 / 60.0) * (V(t + 3) - V(t - 3));
 }
+
+// ducrossensor, part 1 (src/commcal.F90:236-272): ssf of every node; the
+// pressure stencil is clamped at a bounded end (ntype 1 and 2 in the
+// reference, both ends of ntype 4).  GRAD: the velocity gradients are formed
+// here with k_grad_explicit's expression and not stored; whole steps run it
+// where nothing reads the gradients (the inviscid upwind fluxes do not), so
+// that 5 fields move instead of 27; else they are read from dvel.
+// (k_grad_explicit and the sensor from dvel took 80 us at 1025^2 and 85 at
+// 97^3; k_ssf with one node to a load 36 and 41, as it is 21 and 30;
+// 401x337 14 -> 8.3.)
+template <bool GRAD, int ND>
+__global__ __launch_bounds__(256, 4) void k_ssf(SensorArgs a)
+{
+    int c[3];
+    if (!sensor_pair(a, c[0], c[1], c[2])) return;
+    const int i = c[0], n0 = a.g.n[0];
+    const bool two = i < n0;  // node i + 1 exists
+    const unsigned gi = (unsigned)gidx(a.g, i, c[1], c[2]), gb = gi * 8u;
+    double dv[2][9];
+    const double* P = a.prs;
+    const long s1 = a.g.s[1], s2 = a.p2d ? 0 : a.g.s[2];
+    if constexpr (GRAD) {
+        // (past a bounded end the loads meet the halo cells, which exist on
+        // every axis; diff6ec_w leaves them out)
+        double x[3][2];
+#pragma unroll
+        for (int d = 0; d < ND; ++d) {
+            x[d][0] = a.xi[d][c[d] + HM];
+            x[d][1] = d == 0 ? a.xi[0][min(i + 1, n0) + HM] : x[d][0];
+        }
+#pragma unroll
+        for (int m = 0; m < 3; ++m) {
+            const double* f = a.vel[m];
+            const d2 A = ldc2(f - 4, gb), B = ldc2(f - 2, gb), C = ldc2(f, gb);
+            const d2 D = ldc2(f + 2, gb), E = ldc2(f + 4, gb);
+            const double w0[7] = {A.y, B.x, B.y, C.x, C.y, D.x, D.y};
+            const double w1[7] = {B.x, B.y, C.x, C.y, D.x, D.y, E.x};
+            dv[0][3 * m] = diff6ec_w(w0, i, n0, a.ntype[0]) * x[0][0];
+            dv[1][3 * m] = diff6ec_w(w1, i + 1, n0, a.ntype[0]) * x[0][1];
+#pragma unroll
+            for (int d = 1; d < 3; ++d) {
+                if (d >= ND) {
+                    dv[0][3 * m + d] = dv[1][3 * m + d] = 0.0;
+                    continue;
+                }
+                d2 v[7];
+#pragma unroll
+                for (int o = 0; o < 7; ++o) v[o] = o == 3 ? C : ldc2(f + (o - 3) * a.g.s[d], gb);
+#pragma unroll
+                for (int e = 0; e < 2; ++e) {
+                    const double w[7] = {v[0][e], v[1][e], v[2][e], v[3][e], v[4][e], v[5][e], v[6][e]};
+                    dv[e][3 * m + d] = diff6ec_w(w, c[d], a.g.n[d], a.ntype[d]) * x[d][0];
+                }
+            }
+        }
+    } else {
+#pragma unroll
+        for (int m = 0; m < 9; ++m) {
+            const d2 v = ldc2(a.dvel[m], gb);
+            dv[0][m] = v.x;
+            dv[1][m] = v.y;
+        }
+    }
+    const d2 pc = ldc2(P, gb), pl = ldc2(P - 2, gb), pr = ldc2(P + 2, gb);
+    d2 pj1 = ldc2(P + s1, gb), pj0 = ldc2(P - s1, gb), pk1 = ldc2(P + s2, gb), pk0 = ldc2(P - s2, gb);
+    if (hi_end(a.ntype[1]) && c[1] == a.g.n[1]) pj1 = pc;
+    if (lo_end(a.ntype[1]) && c[1] == 0) pj0 = pc;
+    if (hi_end(a.ntype[2]) && c[2] == a.g.n[2]) pk1 = pc;
+    if (lo_end(a.ntype[2]) && c[2] == 0) pk0 = pc;
+    double out[2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+        const double* g = dv[e];
+        const double div = g[0] + g[4] + g[8];
+        const double div2 = div * div;
+        const double vx = g[7] - g[5];  // dvel(3,2) - dvel(2,3)
+        const double vy = g[2] - g[6];  // dvel(1,3) - dvel(3,1)
+        const double vz = g[3] - g[1];  // dvel(2,1) - dvel(1,2)
+        const double vort = vx * vx + vy * vy + vz * vz;
+        const double p0 = pc[e];
+        const double pi1 = hi_end(a.ntype[0]) && i + e == n0 ? p0 : (e == 0 ? pc.y : pr.x);
+        const double pi0 = lo_end(a.ntype[0]) && i + e == 0 ? p0 : (e == 0 ? pl.y : pc.x);
+        const double dpdi = fabs(pi1 - 2.0 * p0 + pi0) / (pi1 + 2.0 * p0 + pi0);
+        const double dpdj = fabs(pj1[e] - 2.0 * p0 + pj0[e]) / (pj1[e] + 2.0 * p0 + pj0[e]);
+        const double dpdk = fabs(pk1[e] - 2.0 * p0 + pk0[e]) / (pk1[e] + 2.0 * p0 + pk0[e]);
+        out[e] = div2 / (div2 + vort + 1.e-30) * uwd::max2(uwd::max2(dpdi, dpdj), dpdk);
+    }
+    if (two) *(d2*)(a.ssf + gi) = d2{out[0], out[1]};
+    else a.ssf[gi] = out[0];
+}
+
+// ducrossensor, part 2 (src/commcal.F90:278-316): lshock = max of ssf over
+// offsets -hm+1..hm along each axis > shkcrt, clamped at bounded ends;
+// along a periodic axis the offsets wrap (dataswap(ssf), src/commcal.F90:
+// 276, src/parallel.F90:4170-4175, which a two-dimensional box's k axis does
+// not need: its planes repeat the plane itself).  (One node to a load ->
+// this: 1025^2 14.2 -> 10.0 us, 97^3 21 -> 16, 401x337 5.4 -> 6.2.)
+__global__ __launch_bounds__(256) void k_ducros_flag(SensorArgs a)
+{
+    int c[3];
+    if (!sensor_pair(a, c[0], c[1], c[2])) return;
+    const int i = c[0], n0 = a.g.n[0];
+    const bool two = i < n0;
+    const unsigned gi = (unsigned)gidx(a.g, i, c[1], c[2]), gb = gi * 8u;
+    const double* f = a.ssf;
+    double m[2] = {0.0, 0.0};
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        if (d >= a.ndims) break;
+        const int n = a.g.n[d], nt = a.ntype[d];
+        const long st = a.g.s[d];
+        if (c[d] >= HM - 1 && c[d] + HM + (d == 0) <= n) {
+            // windows that leave no end of the box, all but a frame of them
+            if (d == 0) {
+                double v[2 * HM + 2];  // i - HM + 1 ..
+#pragma unroll
+                for (int o = 0; o <= HM; ++o) {
+                    const d2 w = ldc2(f + 2 * o - HM + 1, gb);
+                    v[2 * o] = w.x;
+                    v[2 * o + 1] = w.y;
+                }
+#pragma unroll
+                for (int o = 0; o < 2 * HM; ++o) {
+                    m[0] = uwd::max2(m[0], v[o]);
+                    m[1] = uwd::max2(m[1], v[o + 1]);
+                }
+            } else {
+#pragma unroll
+                for (int o = -HM + 1; o <= HM; ++o) {
+                    const d2 w = ldc2(f + o * st, gb);
+                    m[0] = uwd::max2(m[0], w.x);
+                    m[1] = uwd::max2(m[1], w.y);
+                }
+            }
+            continue;
+        }
+        // the frame: the node each offset stands for, every load in flight at
+        // once (a rank's interface end, ntype 1's high and 2's low: the halo,
+        // which no neighbour fills on one domain, is zero)
+#pragma unroll
+        for (int e = 0; e < (d == 0 ? 2 : 1); ++e) {
+            const int t0 = c[d] + e;
+            d2 v[2 * HM];
+#pragma unroll
+            for (int o = 0; o < 2 * HM; ++o) {
+                int t = t0 + o - HM + 1;
+                if (nt == 3) t = t < 0 ? t + n : (t > n ? t - n : t);
+                const int w = min(max(t, 0), n);
+                const bool zero = (t < 0 && !lo_end(nt)) || (t > n && !hi_end(nt));
+                if (d == 0) v[o].x = f[gi + w - i];
+                else v[o] = *(const d2*)(f + gi + (w - t0) * st);
+                if (zero) v[o] = d2{0.0, 0.0};
+            }
+#pragma unroll
+            for (int o = 0; o < 2 * HM; ++o) {
+                m[e] = uwd::max2(m[e], v[o].x);
+                if (d > 0) m[1] = uwd::max2(m[1], v[o].y);
+            }
+        }
+    }
+    a.lshock[gi] = m[0] > a.shkcrt ? 1 : 0;
+    if (two) a.lshock[gi + 1] = m[1] > a.shkcrt ? 1 : 0;
+}
+
+struct GradXArgs {
+    Geo g;
+    int ntype[3], ndims;
+    const double* prim[6];
+    const double* xi[3];
+    double* dvel[9];
+    double* dtmp[3];
+};
 
 // gradcal with the explicit 6th-order derivative (difschm '643e'),
 // src/comsolver.F90:244-497: dvel(m,d) = d/dxi_d(u_m) * dxi(d,d)
@@ -2660,36 +2789,6 @@ __global__ void k_grad_explicit(GradXArgs a)
             else st_nt(&a.dtmp[d][gi], df * x);
         }
     }
-}
-
-// The shock sensor's ssf from the velocity, without storing the gradients:
-// k_grad_explicit's velocity part, then k_ducros_ssf, at one node.  Whole
-// steps run it where nothing reads the gradients (the inviscid upwind
-// fluxes do not): 5 fields move instead of 27.
-// (k_grad_explicit + k_ducros_ssf -> this: 1025^2 80 -> 35 us, 96^3 85 -> 41.)
-__global__ __launch_bounds__(256) void k_grad_ssf(SensorArgs a)
-{
-    const long p = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long ni = a.g.n[0] + 1, nj = a.g.n[1] + 1;
-    if (p >= ni * nj * (a.g.n[2] + 1)) return;
-    int c[3];
-    split3(p, ni, nj, c[0], c[1], c[2]);
-    const long gi = gidx(a.g, c[0], c[1], c[2]);
-    double dv[9];
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        if (d >= a.ndims) {
-#pragma unroll
-            for (int m = 0; m < 3; ++m) dv[3 * m + d] = 0.0;
-            continue;
-        }
-        const long st = a.g.s[d];
-        const double x = a.xi[d][c[d] + HM];
-#pragma unroll
-        for (int m = 0; m < 3; ++m)
-            dv[3 * m + d] = diff6ec_at(a.vel[m] + gi - (long)c[d] * st, st, c[d], a.g.n[d], a.ntype[d]) * x;
-    }
-    a.ssf[gi] = ssf_of(a, c[0], c[1], c[2], gi, dv);
 }
 
 struct FieldXArgs {
@@ -4558,10 +4657,10 @@ int do_sensor(astr_ctx* c, bool fused = false, bool p2d = false)
         a.xi[m] = c->xi + m * c->xi_stride;
     }
     a.p2d = p2d;
-    const long n = n_interior(c);
-    hipLaunchKernelGGL(fused ? k_grad_ssf : k_ducros_ssf, dim3((unsigned)((n + 255) / 256)),
-                       dim3(256), 0, c->stream, a);
-    hipLaunchKernelGGL(k_ducros_flag, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, c->stream, a);
+    const dim3 grid(sensor_layout(a));
+    auto ssf = !fused ? k_ssf<false, 3> : a.ndims == 3 ? k_ssf<true, 3> : k_ssf<true, 2>;
+    hipLaunchKernelGGL(ssf, grid, dim3(256), 0, c->stream, a);
+    hipLaunchKernelGGL(k_ducros_flag, grid, dim3(256), 0, c->stream, a);
     HIPCHK(hipGetLastError());
     return ASTR_OK;
 }
