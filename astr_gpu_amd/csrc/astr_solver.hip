@@ -911,18 +911,26 @@ __device__ __forceinline__ void interior_ijk(const Geo& g, long p, int& i, int& 
 // without FMA contraction (in the reference's operation order, as the
 // upwind checker does)
 #pragma clang fp contract(off)
-__device__ __forceinline__ void q2fvar(const PtArgs& a, const double qv[5], long gi,
-                                       bool write_rho = true)
+__device__ __forceinline__ void prims_of(const PtArgs& a, const double qv[5], double pr[6])
 {
     const double rho = qv[0];
     const double u = qv[1] / rho, v = qv[2] / rho, w = qv[3] / rho;
     const double p = (qv[4] - 0.5 * rho * (u * u + v * v + w * w)) / a.const6;
-    if (write_rho) st_nt(&a.prim[0][gi], rho);
-    st_nt(&a.prim[1][gi], u);
-    st_nt(&a.prim[2][gi], v);
-    st_nt(&a.prim[3][gi], w);
-    st_nt(&a.prim[4][gi], p);
-    st_nt(&a.prim[5][gi], p / rho * a.const2);
+    pr[0] = rho;
+    pr[1] = u;
+    pr[2] = v;
+    pr[3] = w;
+    pr[4] = p;
+    pr[5] = p / rho * a.const2;
+}
+__device__ __forceinline__ void q2fvar(const PtArgs& a, const double qv[5], long gi,
+                                       bool write_rho = true)
+{
+    double pr[6];
+    prims_of(a, qv, pr);
+#pragma unroll
+    for (int m = 0; m < 6; ++m)
+        if (m > 0 || write_rho) st_nt(&a.prim[m][gi], pr[m]);
 }
 #pragma clang fp contract(fast)
 
@@ -942,8 +950,8 @@ __device__ __forceinline__ double miucal(const ViscConst& a, double t)
 }
 
 // qswap of a periodic three-dimensional box, single rank
-// (src/parallel.F90:4877-5200), one kernel per axis in the reference's
-// order:
+// (src/parallel.F90:4877-5200), in the reference's order (k_qswap3 in one
+// launch, the batched queue one part per launch):
 //   i  duplicate nodes q(0) = q(n) = (q(0) + q(n))/2 on every interior row,
 //      then the i-halos copied from the interior before any other average
 //      (src/parallel.F90:4884-4885, 4877-4915);
@@ -952,7 +960,7 @@ __device__ __forceinline__ double miucal(const ViscConst& a, double t)
 //      state.
 // Every halo cell and duplicate node written gets its primitives refreshed
 // (q2fvar); a node that is a duplicate along several axes ends with the
-// primitives of its last average.  Within one kernel the cells read (the
+// primitives of its last average.  Within one part the cells read (the
 // interior sources and the duplicate pairs) and the cells written are
 // disjoint or owned by the same thread, so no thread reads what another
 // writes.
@@ -972,15 +980,10 @@ __device__ __forceinline__ void store_q(const PtArgs& a, long gi, const double (
 // values to make that line whole measured slower, 166 against 102 us per
 // launch at 256^3); lanes 32.. node n and the cells after it to the end of
 // the line of node n+HM (the halo n+1..n+HM from 1..HM, then zeros).
-__device__ __forceinline__ void qswap_x_body(const PtArgs& a, unsigned bid)
+__device__ __forceinline__ void qswap_x_row(const PtArgs& a, unsigned lane, int j, int k, bool avg)
 {
     const Geo& g = a.g;
     const int n0 = g.n[0];
-    const unsigned t = bid * blockDim.x + threadIdx.x;
-    const unsigned row = t / QSX_LANES, lane = t % QSX_LANES;
-    const unsigned nj = (unsigned)g.n[1] + 1;
-    if (row >= nj * ((unsigned)g.n[2] + 1)) return;
-    const int k = (int)(row / nj), j = (int)(row - (unsigned)k * nj);
     int i;
     if (lane < 16) i = (int)lane - 16;
     else if (lane == 16) i = 0;
@@ -989,6 +992,7 @@ __device__ __forceinline__ void qswap_x_body(const PtArgs& a, unsigned bid)
     const long gi = gidx(g, i, j, k);
     double qv[5];
     if (i == 0 || i == n0) {
+        if (!avg) return;
         const long g0 = gidx(g, 0, j, k), gn = gidx(g, n0, j, k);
 #pragma unroll
         for (int m = 0; m < 5; ++m) qv[m] = 0.5 * (a.q[m][g0] + a.q[m][gn]);
@@ -1004,6 +1008,15 @@ __device__ __forceinline__ void qswap_x_body(const PtArgs& a, unsigned bid)
         return;
     }
     store_q(a, gi, qv);
+}
+
+__device__ __forceinline__ void qswap_x_body(const PtArgs& a, unsigned bid)
+{
+    const unsigned t = bid * blockDim.x + threadIdx.x;
+    const unsigned row = t / QSX_LANES, nj = (unsigned)a.g.n[1] + 1;
+    if (row >= nj * ((unsigned)a.g.n[2] + 1)) return;
+    const int k = (int)(row / nj), j = (int)(row - (unsigned)k * nj);
+    qswap_x_row(a, t % QSX_LANES, j, k, true);
 }
 
 // j part (AX = 1) or k part (AX = 2): threads over the nodes i = 0..n of the
@@ -1040,9 +1053,126 @@ __device__ __forceinline__ void qswap_jk_body(const PtArgs& a, unsigned bid)
     store_q(a, at(h), qv);
 }
 
-__global__ __launch_bounds__(256) void k_qswap_x(PtArgs a) { qswap_x_body(a, blockIdx.x); }
-__global__ __launch_bounds__(256) void k_qswap_y(PtArgs a) { qswap_jk_body<1>(a, blockIdx.x); }
-__global__ __launch_bounds__(256) void k_qswap_z(PtArgs a) { qswap_jk_body<2>(a, blockIdx.x); }
+// The three parts in one launch, for the periodic axes among them (a.per; a
+// bounded axis copies nothing).  The averages of the three axes mix only the
+// images of one node (its duplicates 0 and n along every periodic axis it is
+// 0 on), and every halo copy has one source, so a thread that loads all
+// images of a node can write what the three parts write from it: the x halos
+// from the state as it is, the y halos from its x average, the z halos from
+// the y average of that, and the node itself, whose primitives follow its
+// last average.
+//   near blocks: the rows whose j or k sources a halo or is 0 (11 of each
+//     periodic axis), one node per thread, i = 0..n-1 (..n if bounded)
+//   x blocks: of every row that no other average touches (j, k not 0 or n
+//     of a periodic axis) the x halos and, where the row is not near, the
+//     x average: qswap_x_body's lanes
+// No cell is read by one thread and written by another: the x blocks read
+// nodes 1..HM and n-HM..n-1 of rows off the y and z ends, which nothing
+// writes.  n >= 16 > 2 HM keeps an axis's low and high sources apart.
+// (Three launches -> one: 64^3 20.7 -> 13.1 us, 97^3 29 -> 22, 128^3 45 -> 41,
+// 256^3 155 -> 138.)
+struct QsSplit {
+    unsigned near_a, near_b, nb_near;  // near rows by k, by j only; blocks
+    unsigned ri, rj, rk;               // nodes per axis without the duplicate
+    unsigned xrows;                    // rows of the x blocks
+};
+__host__ __device__ inline QsSplit qswap_split(const PtArgs& a)
+{
+    constexpr unsigned NEAR = 2 * HM + 1;
+    QsSplit q;
+    q.ri = (unsigned)(a.g.n[0] + !a.per[0]);
+    q.rj = (unsigned)(a.g.n[1] + !a.per[1]);
+    q.rk = (unsigned)(a.g.n[2] + !a.per[2]);
+    q.near_a = a.per[2] ? NEAR * q.rj : 0;
+    q.near_b = a.per[1] ? NEAR * (q.rk - (a.per[2] ? NEAR : 0)) : 0;
+    q.nb_near = (unsigned)(((long)(q.near_a + q.near_b) * q.ri + 255) / 256);
+    q.xrows = a.per[0] ? (q.rj - (a.per[1] ? 1 : 0)) * (q.rk - (a.per[2] ? 1 : 0)) : 0;
+    return q;
+}
+__global__ __launch_bounds__(256) void k_qswap3(PtArgs a)
+{
+    const Geo& g = a.g;
+    const int n0 = g.n[0], n1 = g.n[1], n2 = g.n[2];
+    const QsSplit sp = qswap_split(a);
+    auto near = [](int c, int n) { return c <= HM || c >= n - HM; };
+    if (blockIdx.x >= sp.nb_near) {
+        const unsigned t = (blockIdx.x - sp.nb_near) * 256 + threadIdx.x;
+        const unsigned row = t / QSX_LANES, lane = t % QSX_LANES;
+        if (row >= sp.xrows) return;
+        const unsigned w = sp.rj - (a.per[1] ? 1 : 0), kk = row / w;
+        const int j = (int)(row - kk * w) + (a.per[1] ? 1 : 0), k = (int)kk + (a.per[2] ? 1 : 0);
+        const bool avg = !(a.per[1] && near(j, n1)) && !(a.per[2] && near(k, n2));
+        qswap_x_row(a, lane, j, k, avg);
+        return;
+    }
+    const unsigned t = blockIdx.x * 256 + threadIdx.x;
+    unsigned r = t / sp.ri;
+    const int i = (int)(t - r * sp.ri);
+    int j, k;
+    if (r < sp.near_a) {
+        k = (int)(r / sp.rj);
+        j = (int)(r - (unsigned)k * sp.rj);
+        if (k > HM) k += n2 - 2 * HM - 1;
+    } else {
+        r -= sp.near_a;
+        if (r >= sp.near_b) return;
+        const unsigned rest = sp.near_b / (2 * HM + 1);
+        j = (int)(r / rest);
+        k = (int)(r - (unsigned)j * rest) + (a.per[2] ? HM + 1 : 0);
+        if (j > HM) j += n1 - 2 * HM - 1;
+    }
+    const bool di = a.per[0] && i == 0, dj = a.per[1] && j == 0, dk = a.per[2] && k == 0;
+    // the halo cell a node sources along a periodic axis (n: none)
+    auto halo = [](int c, int n) { return c >= 1 && c <= HM ? c + n : c >= n - HM && c < n ? c - n : n; };
+    const int hi = a.per[0] ? halo(i, n0) : n0, hj = a.per[1] ? halo(j, n1) : n1;
+    const int hk = a.per[2] ? halo(k, n2) : n2;
+    double f[5], pr[6];
+    // one state to the cells of the images of i and j, or of i
+    auto put = [&](const double (&qv)[5], int ii, int jj, int kk, bool both_i, bool both_j) {
+        prims_of(a, qv, pr);
+#pragma unroll 1
+        for (int e = 0; e < 4; ++e) {
+            if (((e & 1) && !both_i) || ((e & 2) && !both_j)) continue;
+            const long gi = gidx(g, e & 1 ? n0 : ii, e & 2 ? n1 : jj, kk);
+#pragma unroll
+            for (int m = 0; m < 5; ++m) a.q[m][gi] = qv[m];
+#pragma unroll
+            for (int m = 0; m < 6; ++m) st_nt(&a.prim[m][gi], pr[m]);
+        }
+    };
+#pragma unroll
+    for (int ek = 0; ek < 2; ++ek) {
+        if (ek && !dk) break;
+        const int kc = ek ? n2 : k;
+        double v[2][2][5], b[5];  // the images at kc: [j][i]
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int ei = e & 1, ej = e >> 1;
+            if ((ei && !di) || (ej && !dj)) continue;
+            const long gi = gidx(g, ei ? n0 : i, ej ? n1 : j, kc);
+#pragma unroll
+            for (int m = 0; m < 5; ++m) v[ej][ei][m] = a.q[m][gi];
+        }
+#pragma unroll
+        for (int ej = 0; ej < 2; ++ej) {
+            if (ej && !dj) break;
+            if (hi != n0 && (dj || dk)) put(v[ej][0], hi, ej ? n1 : j, kc, false, false);
+            double x[5];
+#pragma unroll
+            for (int m = 0; m < 5; ++m)
+                x[m] = di ? 0.5 * (v[ej][0][m] + v[ej][1][m]) : v[ej][0][m];
+            if (hj != n1) put(x, i, hj, kc, di, false);
+#pragma unroll
+            for (int m = 0; m < 5; ++m) b[m] = ej ? 0.5 * (b[m] + x[m]) : x[m];
+        }
+        if (hk != n2) put(b, i, j, hk, di, dj);
+#pragma unroll
+        for (int m = 0; m < 5; ++m) f[m] = ek ? 0.5 * (f[m] + b[m]) : b[m];
+    }
+    if (!di && !dj && !dk) return;
+    put(f, i, j, k, di, dj);
+    if (dk) put(f, i, j, n2, di, dj);
+}
 
 // threads of the i, j and k parts of a box
 __host__ __device__ inline long qswap_threads(const Geo& g, int axis)
@@ -4410,10 +4540,9 @@ int do_qswap(astr_ctx* c, bool edge = false)
     }
     // each part runs on a periodic axis only (the single-rank branches of
     // qswap copy nothing on a bounded one, src/parallel.F90:4877-4915)
-    if (c->p.npdci == 3) TRY(launch_pt(c, k_qswap_x, qswap_threads(c->g, 0), a));
-    if (c->p.npdcj == 3) TRY(launch_pt(c, k_qswap_y, qswap_threads(c->g, 1), a));
-    if (c->p.npdck == 3) TRY(launch_pt(c, k_qswap_z, qswap_threads(c->g, 2), a));
-    return ASTR_OK;
+    const QsSplit sp = qswap_split(a);
+    const long nb = sp.nb_near + ((long)sp.xrows * QSX_LANES + 255) / 256;
+    return launch_pt(c, k_qswap3, nb * 256, a);
 }
 
 // boucon (src/bc.F90:327-411) for the faces under the user condition of
