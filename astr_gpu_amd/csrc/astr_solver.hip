@@ -1075,25 +1075,52 @@ struct QsSplit {
     unsigned near_a, near_b, nb_near;  // near rows by k, by j only; blocks
     unsigned ri, rj, rk;               // nodes per axis without the duplicate
     unsigned xrows;                    // rows of the x blocks
+    bool py, pz;
 };
-__host__ __device__ inline QsSplit qswap_split(const PtArgs& a)
+__host__ __device__ inline QsSplit qswap_split(const Geo& g, bool px, bool py, bool pz)
 {
     constexpr unsigned NEAR = 2 * HM + 1;
     QsSplit q;
-    q.ri = (unsigned)(a.g.n[0] + !a.per[0]);
-    q.rj = (unsigned)(a.g.n[1] + !a.per[1]);
-    q.rk = (unsigned)(a.g.n[2] + !a.per[2]);
-    q.near_a = a.per[2] ? NEAR * q.rj : 0;
-    q.near_b = a.per[1] ? NEAR * (q.rk - (a.per[2] ? NEAR : 0)) : 0;
+    q.py = py;
+    q.pz = pz;
+    q.ri = (unsigned)(g.n[0] + !px);
+    q.rj = (unsigned)(g.n[1] + !py);
+    q.rk = (unsigned)(g.n[2] + !pz);
+    q.near_a = pz ? NEAR * q.rj : 0;
+    q.near_b = py ? NEAR * (q.rk - (pz ? NEAR : 0)) : 0;
     q.nb_near = (unsigned)(((long)(q.near_a + q.near_b) * q.ri + 255) / 256);
-    q.xrows = a.per[0] ? (q.rj - (a.per[1] ? 1 : 0)) * (q.rk - (a.per[2] ? 1 : 0)) : 0;
+    q.xrows = px ? (q.rj - (py ? 1 : 0)) * (q.rk - (pz ? 1 : 0)) : 0;
     return q;
+}
+// the node (i, j, k) of thread t of the near blocks; i < 0: none
+struct QsNode {
+    int i, j, k;
+};
+__device__ __forceinline__ QsNode qswap_near(const Geo& g, const QsSplit& sp, unsigned t)
+{
+    unsigned r = t / sp.ri;
+    const int i = (int)(t - r * sp.ri);
+    if (r < sp.near_a) {
+        const int k = (int)(r / sp.rj);
+        return {i, (int)(r - (unsigned)k * sp.rj), k > HM ? k + g.n[2] - 2 * HM - 1 : k};
+    }
+    r -= sp.near_a;
+    if (r >= sp.near_b) return {-1, 0, 0};
+    const unsigned rest = sp.near_b / (2 * HM + 1);
+    const int j = (int)(r / rest);
+    return {i, j > HM ? j + g.n[1] - 2 * HM - 1 : j,
+            (int)(r - (unsigned)j * rest) + (sp.pz ? HM + 1 : 0)};
+}
+// the halo cell that node c of a periodic axis of n cells sources (n: none)
+__device__ __forceinline__ int qswap_halo(int c, int n)
+{
+    return c >= 1 && c <= HM ? c + n : c >= n - HM && c < n ? c - n : n;
 }
 __global__ __launch_bounds__(256) void k_qswap3(PtArgs a)
 {
     const Geo& g = a.g;
     const int n0 = g.n[0], n1 = g.n[1], n2 = g.n[2];
-    const QsSplit sp = qswap_split(a);
+    const QsSplit sp = qswap_split(g, a.per[0], a.per[1], a.per[2]);
     auto near = [](int c, int n) { return c <= HM || c >= n - HM; };
     if (blockIdx.x >= sp.nb_near) {
         const unsigned t = (blockIdx.x - sp.nb_near) * 256 + threadIdx.x;
@@ -1105,27 +1132,12 @@ __global__ __launch_bounds__(256) void k_qswap3(PtArgs a)
         qswap_x_row(a, lane, j, k, avg);
         return;
     }
-    const unsigned t = blockIdx.x * 256 + threadIdx.x;
-    unsigned r = t / sp.ri;
-    const int i = (int)(t - r * sp.ri);
-    int j, k;
-    if (r < sp.near_a) {
-        k = (int)(r / sp.rj);
-        j = (int)(r - (unsigned)k * sp.rj);
-        if (k > HM) k += n2 - 2 * HM - 1;
-    } else {
-        r -= sp.near_a;
-        if (r >= sp.near_b) return;
-        const unsigned rest = sp.near_b / (2 * HM + 1);
-        j = (int)(r / rest);
-        k = (int)(r - (unsigned)j * rest) + (a.per[2] ? HM + 1 : 0);
-        if (j > HM) j += n1 - 2 * HM - 1;
-    }
+    const QsNode nd = qswap_near(g, sp, blockIdx.x * 256 + threadIdx.x);
+    const int i = nd.i, j = nd.j, k = nd.k;
+    if (i < 0) return;
     const bool di = a.per[0] && i == 0, dj = a.per[1] && j == 0, dk = a.per[2] && k == 0;
-    // the halo cell a node sources along a periodic axis (n: none)
-    auto halo = [](int c, int n) { return c >= 1 && c <= HM ? c + n : c >= n - HM && c < n ? c - n : n; };
-    const int hi = a.per[0] ? halo(i, n0) : n0, hj = a.per[1] ? halo(j, n1) : n1;
-    const int hk = a.per[2] ? halo(k, n2) : n2;
+    const int hi = a.per[0] ? qswap_halo(i, n0) : n0, hj = a.per[1] ? qswap_halo(j, n1) : n1;
+    const int hk = a.per[2] ? qswap_halo(k, n2) : n2;
     double f[5], pr[6];
     // one state to the cells of the images of i and j, or of i
     auto put = [&](const double (&qv)[5], int ii, int jj, int kk, bool both_i, bool both_j) {
@@ -2179,7 +2191,7 @@ struct AdjArgs {
     double* sb[5];          // qsave-bar
     double const2, const5, const6, reynolds, prandtl, tempconst, tempconst1;
     double rka, rkb, rkc, dt;
-    int stage, axis, visc;
+    int stage, visc;
     double scale;           // 1/(n0 n1 n2) of the statistic
 };
 
@@ -2338,10 +2350,10 @@ __host__ __device__ inline long gflux_adj_halo_count(const Geo& g, int d)
 // the halo node r of axis D's strips (a compile-time axis keeps every
 // index and array in registers)
 template <int D>
-__device__ __forceinline__ void gflux_adj_halo_node(const AdjArgs& a, long r)
+__device__ __forceinline__ void gflux_adj_halo_node(const AdjArgs& a, unsigned r)
 {
     constexpr int OA = D == 0 ? 1 : 0, OB = D == 2 ? 1 : 2;
-    const long ea = a.g.n[OA] + 1L, eb = a.g.n[OB] + 1L;
+    const unsigned ea = (unsigned)a.g.n[OA] + 1, eb = (unsigned)a.g.n[OB] + 1;
     int h, ca, cb;
     if (D == 0) {
         // x strips: the 2 HM halo nodes of a row are the contiguous ones
@@ -2381,9 +2393,9 @@ __global__ void k_gflux_adj_halo(AdjArgs a)
 {
     long r = (long)blockIdx.x * blockDim.x + threadIdx.x;
     const long n0 = gflux_adj_halo_count(a.g, 0), n1 = gflux_adj_halo_count(a.g, 1);
-    if (r < n0) gflux_adj_halo_node<0>(a, r);
-    else if ((r -= n0) < n1) gflux_adj_halo_node<1>(a, r);
-    else if ((r -= n1) < gflux_adj_halo_count(a.g, 2)) gflux_adj_halo_node<2>(a, r);
+    if (r < n0) gflux_adj_halo_node<0>(a, (unsigned)r);
+    else if ((r -= n0) < n1) gflux_adj_halo_node<1>(a, (unsigned)r);
+    else if ((r -= n1) < gflux_adj_halo_count(a.g, 2)) gflux_adj_halo_node<2>(a, (unsigned)r);
 }
 
 // G on the interior reversed at one node: the inviscid parts of its three
@@ -2519,53 +2531,78 @@ __global__ __launch_bounds__(256) void k_gflux_adj_int(AdjArgs a)
     for (int k = 0; k < 6; ++k) st_nt(&a.pb[k][gi], pbv[k]);
 }
 
-// qswap's copies and averages along a.axis reversed, for the lines of that
-// axis over 0..n of the other two: the average q(0) = q(n) = (q(0)+q(n))/2,
-// and the halo copies q(-k) = q(n-k), q(n+k) = q(k).  The eleven pieces
-// touch different nodes (the copies' sources exclude 0 and n), so each is
-// its own thread: op 0 the average, op 1..HM the low halos, HM+1..2HM the
-// high ones.  Run for the axes in the order z, y, x.
-__global__ void k_qswap_adj_line(AdjArgs a)
+// qswap's copies and averages reversed (every axis periodic), along z, y, x:
+// a halo cell's adjoint goes to its source and is cleared, and the images of
+// a duplicate take the mean of theirs.  As in k_qswap3 what a node's images
+// and their halo cells hold concerns no other node, so one thread does the
+// three axes of a node, for one of the five quantities (blockIdx.y): the near
+// blocks as there, and of the other rows the 2 HM + 1 nodes of the x ends.
+// (A launch per axis, one piece of a line per thread, and 64-bit index
+// arithmetic before: 80x64x72 54 -> 10.5 us.)
+__global__ __launch_bounds__(256) void k_qswap_adj(AdjArgs a)
 {
-    const int d = a.axis;
-    const long ext[3] = {a.g.n[0] + 1, a.g.n[1] + 1, a.g.n[2] + 1};
-    const int oa = d == 0 ? 1 : 0, ob = d == 2 ? 1 : 2;
-    const long nl = ext[oa] * ext[ob];
-    long r = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= (2 * HM + 1) * 5 * nl) return;
-    int op, m;
-    if (d == 0) {
-        // x lines: the pieces of one row are neighbours (the same lines)
-        op = (int)(r % (2 * HM + 1));
-        r /= 2 * HM + 1;
-        m = (int)(r % 5);
-        r /= 5;
+    const Geo& g = a.g;
+    const int n0 = g.n[0], n1 = g.n[1], n2 = g.n[2];
+    const QsSplit sp = qswap_split(g, true, true, true);
+    QsNode nd;
+    if (blockIdx.x >= sp.nb_near) {
+        const unsigned t = (blockIdx.x - sp.nb_near) * 256 + threadIdx.x;
+        const unsigned row = t / 16, w = sp.rj - (2 * HM + 1), kk = row / w;
+        const int i = (int)(t % 16);
+        nd = {i > HM ? i + n0 - 2 * HM - 1 : i, (int)(row - kk * w) + HM + 1, (int)kk + HM + 1};
+        if (i > 2 * HM || nd.k >= n2 - HM) return;
     } else {
-        // y and z lines: neighbouring threads take neighbouring i
-        op = (int)(r / (5 * nl));
-        r -= op * 5 * nl;
-        m = (int)(r / nl);
-        r -= m * nl;
+        nd = qswap_near(g, sp, blockIdx.x * 256 + threadIdx.x);
+        if (nd.i < 0) return;
     }
-    int c[3];
-    c[oa] = (int)(r % ext[oa]);
-    c[ob] = (int)(r / ext[oa]);
-    c[d] = 0;
-    const long sd = a.g.s[d];
-    const int n = a.g.n[d];
-    double* f = a.qb[m] + gidx(a.g, c[0], c[1], c[2]);
-    if (op == 0) {
-        const double t = f[0] + f[n * sd];
-        f[0] = 0.5 * t;
-        f[n * sd] = 0.5 * t;
-    } else if (op <= HM) {
-        const int k = op;
-        f[(n - k) * sd] += f[-k * sd];
-        f[-k * sd] = 0.0;
-    } else {
-        const int k = op - HM;
-        f[k * sd] += f[(n + k) * sd];
-        f[(n + k) * sd] = 0.0;
+    const int i = nd.i, j = nd.j, k = nd.k;
+    double* f = a.qb[blockIdx.y];
+    const bool di = i == 0, dj = j == 0, dk = k == 0;
+    const int hi = qswap_halo(i, n0), hj = qswap_halo(j, n1), hk = qswap_halo(k, n2);
+    auto at = [&](int ei, int ej, int ek) { return gidx(g, ei ? n0 : i, ej ? n1 : j, ek ? n2 : k); };
+    // the images [k][j][i] and the halo cells they source
+    double v[2][2][2], hz[2][2], hy[2][2], hx[2][2];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const int ei = e & 1, ej = (e >> 1) & 1, ek = e >> 2;
+        v[ek][ej][ei] = (ei && !di) || (ej && !dj) || (ek && !dk) ? 0.0 : f[at(ei, ej, ek)];
+    }
+    auto take = [&](bool on, int ci, int cj, int ck) {
+        if (!on) return 0.0;
+        const long gi = gidx(g, ci, cj, ck);
+        const double h = f[gi];
+        f[gi] = 0.0;
+        return h;
+    };
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const int p = e & 1, q = e >> 1;  // the images of the two other axes, the first in p
+        hz[q][p] = take(hk != n2 && (!p || di) && (!q || dj), p ? n0 : i, q ? n1 : j, hk);
+        hy[q][p] = take(hj != n1 && (!p || di) && (!q || dk), p ? n0 : i, hj, q ? n2 : k);
+        hx[q][p] = take(hi != n0 && (!p || dj) && (!q || dk), hi, p ? n1 : j, q ? n2 : k);
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const int p = e & 1, q = e >> 1;
+        if (hk != n2) v[0][q][p] += hz[q][p];
+        if (dk) v[0][q][p] = v[1][q][p] = 0.5 * (v[0][q][p] + v[1][q][p]);
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const int p = e & 1, q = e >> 1;
+        if (hj != n1) v[q][0][p] += hy[q][p];
+        if (dj) v[q][0][p] = v[q][1][p] = 0.5 * (v[q][0][p] + v[q][1][p]);
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const int p = e & 1, q = e >> 1;
+        if (hi != n0) v[q][p][0] += hx[q][p];
+        if (di) v[q][p][0] = v[q][p][1] = 0.5 * (v[q][p][0] + v[q][p][1]);
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const int ei = e & 1, ej = (e >> 1) & 1, ek = e >> 2;
+        if (!((ei && !di) || (ej && !dj) || (ek && !dk))) f[at(ei, ej, ek)] = v[ek][ej][ei];
     }
 }
 
@@ -4540,7 +4577,7 @@ int do_qswap(astr_ctx* c, bool edge = false)
     }
     // each part runs on a periodic axis only (the single-rank branches of
     // qswap copy nothing on a bounded one, src/parallel.F90:4877-4915)
-    const QsSplit sp = qswap_split(a);
+    const QsSplit sp = qswap_split(a.g, a.per[0], a.per[1], a.per[2]);
     const long nb = sp.nb_near + ((long)sp.xrows * QSX_LANES + 255) / 256;
     return launch_pt(c, k_qswap3, nb * 256, a);
 }
@@ -5575,12 +5612,11 @@ int qswap_adj(astr_ctx* c, AdjArgs a)
 {
     hipLaunchKernelGGL(k_q2f_adj, padded_grid(c), dim3(256), 0, c->stream, a);
     HIPCHK(hipGetLastError());
-    const long ext[3] = {c->g.n[0] + 1L, c->g.n[1] + 1L, c->g.n[2] + 1L};
-    for (int d = 2; d >= 0; --d) {
-        a.axis = d;
-        const long nl = d == 0 ? ext[1] * ext[2] : d == 1 ? ext[0] * ext[2] : ext[0] * ext[1];
-        TRY(launch_adj(c, k_qswap_adj_line, (2 * HM + 1) * 5 * nl, a));
-    }
+    const QsSplit sp = qswap_split(c->g, true, true, true);
+    const long xrows = (long)(sp.rj - 2 * HM - 1) * (sp.rk - 2 * HM - 1);
+    const dim3 grid(sp.nb_near + (unsigned)((xrows * 16 + 255) / 256), 5);
+    hipLaunchKernelGGL(k_qswap_adj, grid, dim3(256), 0, c->stream, a);
+    HIPCHK(hipGetLastError());
     return ASTR_OK;
 }
 

@@ -67,7 +67,7 @@ FAMILY_DOUBLES = {
 FAMILY_KERNEL = {"filter": "k_sweep<L,0> (filter)", "grad": "k_sweep<L,1> (y and z gradient)",
                  "gflux": "k_row_flux<L> (x gradient, fluxes, x flux derivative)", "flux": "k_sweep<L,2> (flux derivatives, RK3 in z)",
                  "prim": "k_prim"}
-FAMILY_LAUNCHES = {"filter": 3, "qswap": 2, "grad": 2, "gflux": 1, "stats": 0, "flux": 2,
+FAMILY_LAUNCHES = {"filter": 3, "qswap": 1, "grad": 2, "gflux": 1, "stats": 0, "flux": 2,
                    "prim": 1}
 FAMILY_NAMES = ["filter", "qswap", "grad", "gflux", "stats", "flux", "prim"]
 STATS_DOUBLES = 1.0  # the statistics' rho, loaded by stage 1's k_row_flux

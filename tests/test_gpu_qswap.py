@@ -7,6 +7,7 @@ import numpy as np
 import pytest
 
 import astr_gpu_amd as ag
+from test_gpu_adjoint import test_adjoint_matches_torch_autograd as adjoint_matches
 
 pytestmark = pytest.mark.gpu
 HM = 5
@@ -75,3 +76,10 @@ def test_one_launch_equals_the_parts(dims, npdc):
     rest[:, :HM] = rest[:, -HM:] = rest[:, :, :HM] = rest[:, :, -HM:] = False
     for k, v in (("rho", 1.0), ("prs", 3.0), ("tmp", 4.0)):
         assert np.all(g[k][rest] == v)
+
+
+@pytest.mark.parametrize("dims", [(16, 16, 16), (17, 23, 16), (34, 17, 19)])
+def test_reversal_in_one_launch(dims):
+    """The reversed parts in one launch, inside the whole reversal, against
+    PyTorch's autograd of the same forward (its own bounds)."""
+    adjoint_matches(1, 1, None, dims)
