@@ -911,7 +911,8 @@ __device__ __forceinline__ void interior_ijk(const Geo& g, long p, int& i, int& 
 // without FMA contraction (in the reference's operation order, as the
 // upwind checker does)
 #pragma clang fp contract(off)
-__device__ __forceinline__ void prims_of(const PtArgs& a, const double qv[5], double pr[6])
+template <class A>
+__device__ __forceinline__ void prims_of(const A& a, const double qv[5], double pr[6])
 {
     const double rho = qv[0];
     const double u = qv[1] / rho, v = qv[2] / rho, w = qv[3] / rho;
@@ -3579,6 +3580,88 @@ __global__ void k_bc_riem2d_j(BcArgs a)
         }
     }
 }
+
+// The same for the four faces of udf_bc in one launch, one thread per
+// node of the rim of a plane k: where k_bc_riem2d_j would read what
+// k_bc_riem2d_i has just written (its column i = 0) it forms that value
+// itself, and the rest it reads is inside the rim.  refresh: the primitives
+// are left as q2fvar gives them from the q set here, which the k part of
+// qswap would do to the rim next.
+// (Two launches and k_qswap2d_edge -> one: 401x337 16.4 -> 5.1 us a stage.)
+__global__ void k_bc_riem2d(BcArgs a, int refresh)
+{
+    const int im = a.g.n[0], jm = a.g.n[1], ni = im + 1;
+    const unsigned rim = 2u * (unsigned)(im + jm);
+    const unsigned t = blockIdx.x * blockDim.x + threadIdx.x;
+    const int k = (int)(t / rim), s = (int)(t - (unsigned)k * rim);
+    if (k > a.g.n[2]) return;
+    const int i = s < 2 * ni ? s % ni : (s - 2 * ni) % 2 * im;
+    const int j = s < 2 * ni ? s / ni * jm : 1 + (s - 2 * ni) / 2;
+    R2D_STATES
+    const double n1d3 = 1.0 / 3.0;
+    double r, u, v, p;
+    auto face1 = [&](int jj, double& r1, double& p1) {  // behind or ahead of the shock at x = 0
+        const double t1 = p01 / r01 * a.const2;
+        const double vss = shockspeed(a, p01, t1, p00);
+        const double ys = 0.8 - vss * a.time;
+        const bool up = (1.0 / (double)jm) * (double)jj > ys;
+        r1 = up ? r01 : r00;
+        p1 = up ? p01 : p00;
+        return up ? v01 : v00;
+    };
+    if (j == 0) {
+        const double t1 = p10 / r10 * a.const2;
+        const double vss = shockspeed(a, p10, t1, p00);
+        const double xs = 0.8 - vss * a.time;
+        const bool up = (1.0 / (double)im) * (double)i > xs;
+        r = up ? r10 : r00;
+        u = up ? u10 : u00;
+        v = v10;
+        p = up ? p10 : p00;
+    } else if (i == im && j == jm) {
+        r = r11;
+        u = 0.0;
+        v = 0.0;
+        p = p11;
+    } else if (j == jm) {
+        double ra, pa, rb, pb, ua = u01, ub = u01;
+        if (i == 0) {
+            face1(jm - 1, ra, pa);
+            face1(jm - 2, rb, pb);
+        } else {
+            const long g1 = gidx(a.g, i, jm - 1, k), g2 = gidx(a.g, i, jm - 2, k);
+            ra = a.prim[0][g1], rb = a.prim[0][g2];
+            pa = a.prim[4][g1], pb = a.prim[4][g2];
+            ua = a.prim[1][g1], ub = a.prim[1][g2];
+        }
+        r = n1d3 * (4.0 * ra - rb);
+        p = n1d3 * (4.0 * pa - pb);
+        u = n1d3 * (4.0 * ua - ub);
+        v = 0.0;
+    } else if (i == 0) {
+        v = face1(j, r, p);
+        u = u01;
+    } else {
+        const long g1 = gidx(a.g, im - 1, j, k), g2 = gidx(a.g, im - 2, j, k);
+        r = n1d3 * (4.0 * a.prim[0][g1] - a.prim[0][g2]);
+        p = n1d3 * (4.0 * a.prim[4][g1] - a.prim[4][g2]);
+        v = n1d3 * (4.0 * a.prim[2][g1] - a.prim[2][g2]);
+        u = 0.0;
+    }
+    (void)v11;
+    const long gi = gidx(a.g, i, j, k);
+    if (!refresh) {
+        bc_node(a, gi, r, u, v, 0.0, p);
+        return;
+    }
+    const double qv[5] = {r, r * u, r * v, r * 0.0, p * a.const6 + r * (0.5 * (u * u + v * v + 0.0 * 0.0))};
+    double pr[6];
+    prims_of(a, qv, pr);
+#pragma unroll
+    for (int m = 0; m < 5; ++m) a.q[m][gi] = qv[m];
+#pragma unroll
+    for (int m = 0; m < 6; ++m) a.prim[m][gi] = pr[m];
+}
 #undef R2D_STATES
 
 // gcnscbc (bctype 23), src/bc.F90:7907-8137: the ghost-cell NSCBC of
@@ -4604,13 +4687,18 @@ static int launch_extrap(astr_ctx* c, const BcArgs& a, int f)
     return ASTR_OK;
 }
 
-int do_boucon(astr_ctx* c)
+// rim: whether, where one launch sets the whole rim of a two-dimensional
+// box, it refreshes the rim's primitives as well; set to whether it did
+int do_boucon(astr_ctx* c, bool* rim = nullptr)
 {
+    const bool refresh = rim && *rim;
+    if (rim) *rim = false;
     bool any = c->udf == ASTR_UDF_RIEMANN2D;
-    for (int f = 0; f < 6; ++f)
-        any = any || c->bctype[f] == 50 || c->bctype[f] == 60 || c->bctype[f] == 23 ||
-              c->bctype[f] == 41 || c->bctype[f] == 42 || c->bctype[f] == 21 ||
-              c->bctype[f] == 31 || c->bctype[f] == 421 || c->bctype[f] == 411;
+    auto bc_set = [](int t) {
+        return t == 50 || t == 60 || t == 23 || t == 41 || t == 42 || t == 21 || t == 31 ||
+               t == 421 || t == 411;
+    };
+    for (int f = 0; f < 6; ++f) any = any || bc_set(c->bctype[f]);
     if (!any) return ASTR_OK;
     BcArgs a{};
     a.g = c->g;
@@ -4634,7 +4722,16 @@ int do_boucon(astr_ctx* c)
     // zeroextrap and symmetry on any
     const long nk = c->g.n[2] + 1;
     const long ni = (long)(c->g.n[0] + 1) * nk, nj = (long)(c->g.n[1] + 1) * nk;
-    for (int f = 0; f < 6; ++f) {
+    const bool all = a.face[0] && a.face[1] && a.face[2] && a.face[3];
+    if (all) {
+        const bool last = !bc_set(c->bctype[4]) && !bc_set(c->bctype[5]);
+        const long nt = 2L * (c->g.n[0] + c->g.n[1]) * nk;
+        hipLaunchKernelGGL(k_bc_riem2d, dim3((unsigned)((nt + 63) / 64)), dim3(64), 0, c->stream, a,
+                           (int)(refresh && last));
+        HIPCHK(hipGetLastError());
+        if (refresh && last) *rim = true;
+    }
+    for (int f = all ? 4 : 0; f < 6; ++f) {
         if (f == 0 && (a.face[0] || a.face[1])) {
             hipLaunchKernelGGL(k_bc_riem2d_i, dim3((unsigned)((nj + 255) / 256)), dim3(256), 0,
                                c->stream, a);
@@ -5338,12 +5435,13 @@ int do_step(astr_ctx* c, double dt, double* stats_slot, bool timed, bool alt = f
         if (timed) TRY(time_mark(c, 1));
         // boucon before qswap (src/mainloop.F90:413-415), at the step's
         // start time in every stage
-        TRY(do_boucon(c));
         // (where a call begins or ends the whole plane: the primitives may
         // not be q's yet, and the pressure planes are left for the host)
         const bool ends = (s == 1 && first) || (s == 3 && last);
         const bool edge = upwind && c->g.n[2] == 0 && !ends;
-        TRY(do_qswap(c, edge));
+        bool rim = edge && c->p.npdci != 3 && c->p.npdcj != 3;
+        TRY(do_boucon(c, &rim));
+        if (!rim) TRY(do_qswap(c, edge));
         if (timed) TRY(time_mark(c, 2));
         // rkfirst's statcal sees the stage-1 state and its gradients; the
         // central path sums it with the fluxes, which load the same inputs
