@@ -4279,6 +4279,25 @@ std::vector<std::pair<int, double>> b_closure_row(int op, int ntype, int first, 
     return v;
 }
 
+// The filter's closure rows as the line engine takes them: 32 rows of CLS
+// coefficients (lane sub's row; the lanes between the ends unused)
+std::vector<double> build_closure(int ntype, const HostTab& h, const FiltCoef& f, LineTab& t)
+{
+    const bool lob = ntype == 1 || ntype == 4, hib = ntype == 2 || ntype == 4;
+    t.nlo = lob ? 5 : 3;
+    t.nhi = hib ? 5 : 3;
+    t.clo = lob ? h.first : h.first - 2;
+    t.chi = hib ? h.last : h.last + 2;
+    std::vector<double> cl(32 * CLS, 0.0);
+    for (int r = 0; r < t.nlo; ++r)
+        for (const auto& e : b_closure_row(OP_FILTER, ntype, h.first, h.last, h.R, r, f))
+            cl[CLS * r + (e.first - t.clo)] += e.second;
+    for (int k = 0; k < t.nhi; ++k)
+        for (const auto& e : b_closure_row(OP_FILTER, ntype, h.first, h.last, h.R, h.R - 1 - k, f))
+            cl[CLS * (31 - k) + (t.chi - e.first)] += e.second;
+    return cl;
+}
+
 // The closure-correction blocks of B^T for one line system: nlo rows at the
 // low end (columns first-5 ..), nhi at the high end (columns last-10 ..)
 void build_trans_blocks(int op, int ntype, const HostTab& h, const FiltCoef& f, int& nlo, int& nhi,
@@ -6281,8 +6300,10 @@ int astr_create(const astr_params* p, int32_t device, astr_ctx** out)
     c->tempconst1 = 1.0 + c->tempconst;
 
     // line systems
+    const FiltCoef fc = build_coef(p->alfa_filter, p->beta_halo, p->beta_bound);
     std::vector<double> tabs;
     std::vector<long> offs;
+    long cloffs[3] = {};
     for (int d = 0; d < 3; ++d) {
         // an axis the compact sweeps cannot take (the k axis of a 2-D box, a
         // long axis of an upwind context) keeps the line systems of a
@@ -6301,6 +6322,11 @@ int astr_create(const astr_params* p, int32_t device, astr_ctx** out)
             t.dim = dims[d];
             t.op = op;
             t.L = c->L[d];
+            if (op != OP_FILTER) continue;
+            const std::vector<double> cl = build_closure(nts[d], h, fc, t);
+            if (tabs.size() % 2) tabs.push_back(0.0);  // 16-byte loads
+            cloffs[d] = (long)tabs.size();
+            tabs.insert(tabs.end(), cl.begin(), cl.end());
         }
     }
     if (hipMalloc(&c->tabs, sizeof(double) * tabs.size()) != hipSuccess)
@@ -6308,7 +6334,10 @@ int astr_create(const astr_params* p, int32_t device, astr_ctx** out)
     if (hipMemcpy(c->tabs, tabs.data(), sizeof(double) * tabs.size(), hipMemcpyHostToDevice) != hipSuccess)
         return cleanup(fail(ASTR_E_HIP, "table copy failed"));
     for (int d = 0, s = 0; d < 3; ++d)
-        for (int op = 0; op < 2; ++op, ++s) c->tab[d][op].t = c->tabs + offs[s];
+        for (int op = 0; op < 2; ++op, ++s) {
+            c->tab[d][op].t = c->tabs + offs[s];
+            if (op == OP_FILTER) c->tab[d][op].cl = c->tabs + cloffs[d];
+        }
 
     if (p->convection == 2)
         for (int d = 0; d < (two_d ? 2 : 3); ++d)
@@ -6320,7 +6349,6 @@ int astr_create(const astr_params* p, int32_t device, astr_ctx** out)
                               hipMemcpyHostToDevice) != hipSuccess)
                     return cleanup(fail(ASTR_E_HIP, "compact flux table upload failed"));
             }
-    FiltCoef fc = build_coef(p->alfa_filter, p->beta_halo, p->beta_bound);
     if (hipMalloc(&c->fc, sizeof(FiltCoef)) != hipSuccess ||
         hipMemcpy(c->fc, &fc, sizeof fc, hipMemcpyHostToDevice) != hipSuccess)
         return cleanup(fail(ASTR_E_HIP, "coefficient upload failed"));

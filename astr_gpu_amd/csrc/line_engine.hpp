@@ -20,7 +20,10 @@
 // once.  The filter's closure rows at the low end of a line without a
 // boundary there (the 11-point halo rows) are evaluated by lane 0 from its
 // window; the other closure rows are evaluated wave-uniformly (scalar
-// coefficient loads) and handed to the lane that owns them.
+// coefficient loads) and handed to the lane that owns them.  On short lines
+// the filter's closure rows are evaluated one per lane instead, with the
+// coefficients from a table, and reach their owners through the line's LDS
+// slots.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -41,9 +44,22 @@ struct LineTab {
     int dim;    // line nodes 0..dim
     int op;     // LineOp
     int L;      // rows per lane
-    int pad;
+    // filter: the closure rows at each end (nlo, nhi of them) as dot products
+    // of CLW nodes: row r at the low end over the nodes clo, clo + 1, ..,
+    // row R-1-k at the high end over chi, chi - 1, ..; coefficients cl[CLS r]
+    // for the low rows, cl[CLS (31 - k)] for the high ones
+    int nlo, nhi, clo, chi;
     const double* __restrict__ t;
+    const double* __restrict__ cl;
 };
+constexpr int CLW = 11, CLS = 12;  // width of a closure row, its stride in cl
+constexpr int CLR = 5;             // most closure rows at an end
+// Rows per lane up to which the filter's closure rows are taken one per lane
+// (below).  Per launch: 64^3 (L = 3) y/z 17.7 -> 15.4 us and x 13.8 -> 12.4,
+// 112x81x64 y/z 30.4 -> 25.8, 40x32x36 (L = 2) 9.9 -> 7.1; at L = 5
+// (128^3) 56 -> 63 and at L = 9 (256^3) 320 -> 372: there the rows after each
+// other hide behind the other wavefronts' loads, and the table's do not.
+constexpr int CL_LANES_MAX = 3;
 
 // filter_coefficient_cal tables (src/filter.F90:299-432) used on the path.
 struct FiltCoef {
@@ -237,12 +253,12 @@ __device__ __forceinline__ void solve_line(const double* ln, const LineTab& tb,
             if constexpr (OP == OP_DERIV) x[t] = rhs_deriv_in(w + t + HW);
             else x[t] = rhs_filter_in(w + t + HW, fc);
         }
-        if constexpr (OP == OP_FILTER && L >= 4) {
+        if constexpr (OP == OP_FILTER && L > CL_LANES_MAX) {
             // The closure rows at the low end of a line without a boundary
             // there (the 11-point ch rows of compact_filter_rhs) from lane
             // 0's window, in the reference's summation order: rows 0..2 are
-            // its x[0..2], and the window (nodes first-5..first+L+4, so
-            // L >= 4) holds their nodes first-2..first+8 at w[3..13].  (The
+            // its x[0..2], and the window (nodes first-5..first+L+4, L >= 4)
+            // holds their nodes first-2..first+8 at w[3..13].  (The
             // high end's rows sit at a run-time place in their owner's
             // window and are taken from LDS below.)
             if (!lo_boundary(tb.ntype) && sub == 0) {
@@ -256,8 +272,40 @@ __device__ __forceinline__ void solve_line(const double* ln, const LineTab& tb,
             }
         }
     }
-    // the closure rows at both ends, computed wave-uniformly
-    if constexpr (OP == OP_DERIV) {
+    // the closure rows at both ends: the filter's on short lines one per lane,
+    // the others computed wave-uniformly
+    if constexpr (OP == OP_FILTER && L <= CL_LANES_MAX) {
+        // (compact_filter_rhs, src/filter.F90:176-264) low row sub on lane
+        // sub, high row R-1-k on lane 31-k: one dot product for all of them.
+        // (Row after row, each a chain of scalar coefficient loads and
+        // branches on the closure type, they took half the solve of a short
+        // line.)
+        double cv = 0.0;
+        if (sub < tb.nlo || 31 - sub < tb.nhi) {
+            const bool lo = sub < CLR;
+            const double* c = tb.cl + CLS * sub;
+            const double* f = ln + HM + (lo ? tb.clo : tb.chi);
+            const int st = lo ? 1 : -1;
+#pragma unroll
+            for (int j = 0; j < CLW; ++j) cv = fma(c[j], f[st * j], cv);
+        }
+        // Every lane has read its window (and its closure row's nodes): the
+        // closure values go into their rows' slots of the line, which the
+        // solution overwrites, and the owners take them from there.
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        double* row = const_cast<double*>(ln) + HM + tb.first;
+        if (sub < tb.nlo) row[sub] = cv;
+        if (31 - sub < tb.nhi) row[R - 1 - (31 - sub)] = cv;
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int r = 0; r < CLR; ++r)
+            if (r < tb.nlo) set_row(x, r, sub, row[r]);
+#pragma unroll
+        for (int k = 0; k < CLR; ++k)
+            if (k < tb.nhi) set_row(x, R - 1 - k, sub, row[R - 1 - k]);
+    } else if constexpr (OP == OP_DERIV) {
         const int ne = (lo_boundary(tb.ntype) ? 2 : 1);
 #pragma unroll
         for (int j = 0; j < 2; ++j)
@@ -268,10 +316,8 @@ __device__ __forceinline__ void solve_line(const double* ln, const LineTab& tb,
             set_row(x, r, sub, rhs_deriv_edge(ln + HM + tb.first + r, r, tb));
         }
     } else {
-        // boundary closures, and the halo closure rows the windows above
-        // did not give
-        const bool lo_done = L >= 4 && !lo_boundary(tb.ntype);
-        const int ne = lo_boundary(tb.ntype) ? 5 : (lo_done ? 0 : 3);
+        // boundary closures, and the high end's halo closure rows
+        const int ne = lo_boundary(tb.ntype) ? 5 : 0;
 #pragma unroll
         for (int r = 0; r < 5; ++r)
             if (r < ne) set_row(x, r, sub, rhs_filter_edge(ln, r, tb, fc));
