@@ -37,7 +37,9 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <memory>
 #include <mutex>
+#include <new>
 #include <string>
 #include <thread>
 #include <type_traits>
@@ -5300,8 +5302,15 @@ int transfer(astr_ctx* c, const std::vector<HostField>& fields, bool up)
     // of a 97x65x81 field, 7 MB up and down: 1 worker 0.51 ms, 4 0.79.)
     const int want = (int)std::min<double>(XFER_THREADS, std::max(1.0, std::sqrt(bytes / 2e6)));
     std::vector<PinBuf*> bufs = pin_take(want);
-    if (bufs.empty()) return fail(ASTR_E_NOMEM, "pinned host buffer");
-    const int nw = (int)bufs.size();
+    // where pinned memory is refused, one worker through plain memory
+    PinBuf plain;
+    std::unique_ptr<double[]> mem;
+    if (bufs.empty()) {
+        mem.reset(new (std::nothrow) double[2 * PIN_HALF / sizeof(double)]);
+        if (!mem) return fail(ASTR_E_NOMEM, "host buffer");
+        plain.p = mem.get();
+    }
+    const int nw = std::max(1, (int)bufs.size());
     // chunks of at most a half, and a few for each worker's two halves
     const long chunk = std::max<long>(
         std::min<long>((long)(PIN_HALF / sizeof(double)), (total / nw + 3) / 4), 1 << 16);
@@ -5366,9 +5375,10 @@ int transfer(astr_ctx* c, const std::vector<HostField>& fields, bool up)
     } catch (...) {
         // no more threads: the ones that started, and this one, do the work
     }
-    work(bufs[0]);
+    work(mem ? &plain : bufs[0]);
     for (std::thread& t : ts) t.join();
-    pin_give(bufs);
+    plain.p = nullptr;  // not the pool's to free
+    if (!mem) pin_give(bufs);
     if (err != (int)hipSuccess)
         return fail(ASTR_E_HIP, std::string("host transfer: ") + hipGetErrorString((hipError_t)err.load()));
     return ASTR_OK;
