@@ -50,7 +50,7 @@ HBM_PEAK_GBS = 8000.0
 FAMILY_DOUBLES = {
     "filter": 10.0,   # q(1:5) in and out, per axis
     "qswap": None,    # boundary planes only
-    "grad": 8.0,      # u, v, w, T in; dvel(.,d), dtmp(d) out
+    "grad": 16.0,     # y and z: each u, v, w, T in; dvel(.,d), dtmp(d) out
     # u, v, w, T, p, q 5 and the y and z gradients (8) in; the fluxes G of y
     # and z (2 x 5) and the x derivative of G_x in qrhs (5) out (a grid whose
     # Jacobian varies also reads J; the box's is one scalar)
@@ -64,10 +64,10 @@ FAMILY_DOUBLES = {
     # the density in between)
     "prim": (10.0 + 10.0 + 11.0) / 3.0,
 }
-FAMILY_KERNEL = {"filter": "k_sweep<L,0> (filter)", "grad": "k_sweep<L,1> (y and z gradient)",
+FAMILY_KERNEL = {"filter": "k_sweep<L,0> (filter)", "grad": "k_sweep_grad_yz<L> (y and z gradient)",
                  "gflux": "k_row_flux<L> (x gradient, fluxes, x flux derivative)", "flux": "k_sweep<L,2> (flux derivatives, RK3 in z)",
                  "prim": "k_prim"}
-FAMILY_LAUNCHES = {"filter": 3, "qswap": 1, "grad": 2, "gflux": 1, "stats": 0, "flux": 2,
+FAMILY_LAUNCHES = {"filter": 3, "qswap": 1, "grad": 1, "gflux": 1, "stats": 0, "flux": 2,
                    "prim": 1}
 FAMILY_NAMES = ["filter", "qswap", "grad", "gflux", "stats", "flux", "prim"]
 STATS_DOUBLES = 1.0  # the statistics' rho, loaded by stage 1's k_row_flux
