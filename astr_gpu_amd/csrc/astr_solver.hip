@@ -4850,11 +4850,13 @@ int do_boucon(astr_ctx* c, bool* rim = nullptr)
 // primitives.
 const double RKC[3][3] = {{1.0, 0.0, 1.0}, {0.75, 0.25, 0.25}, {1.0 / 3.0, 2.0 / 3.0, 2.0 / 3.0}};
 
-// viscous flow on rectilinear metrics: the x part of the gradient and of
-// the flux derivative runs with the fluxes in k_row_flux
+// viscous flow on rectilinear metrics with the compact gradient: the x part
+// of the gradient and of the flux derivative runs with the fluxes in
+// k_row_flux (whose gradient is the compact one: with the explicit gradient
+// only the fluxes are differentiated so)
 bool row_flux_ok(const astr_ctx* c)
 {
-    return !c->curv && c->p.diffterm != 0 && c->p.variant == 0;
+    return !c->curv && c->p.diffterm != 0 && c->p.variant == 0 && !c->p.deriv_explicit;
 }
 
 int do_flux_sweeps(astr_ctx* c, int rk_stage, double dt, double* const* qo = nullptr,
@@ -4913,8 +4915,8 @@ int do_gflux(astr_ctx* c, double* stats_slot = nullptr)
 // also stores the x gradients (what the statistics, the reversal and
 // astr_download_rhs read).  General metrics combine the three axes'
 // derivatives before the fluxes, so they keep the separate launches, as do
-// the mini-app's forms and inviscid flow.  mark: the timing slot between the
-// gradient and the fluxes.
+// the mini-app's forms, inviscid flow and the explicit gradient.  mark: the
+// timing slot between the gradient and the fluxes.
 int do_grad(astr_ctx* c);
 int time_mark(astr_ctx* c, int slot);
 int do_central_flux(astr_ctx* c, bool keep_grad, double* stats_slot = nullptr, int mark = -1)
