@@ -472,8 +472,8 @@ __device__ __forceinline__ void sweep_tile(const A& args, const A& args_w, int t
     // LDS row holds.
     const bool dead = PASS == PASS_GRAD || (PASS == PASS_RHS && (XD || a.rk_stage == 0));
     // the RK3 combine of the z sweep stores q unchanged on those lines; the
-    // y/z filter stages those lines themselves, leaves them unsolved and
-    // stores them back as staged
+    // y/z filter stages those lines themselves, leaves them in LDS as they
+    // are and stores them back
     const bool keepq = PASS == PASS_RHS && !XD && a.rk_stage != 0;
     const bool keepf = PASS == PASS_FILTER && !XD;
     const bool lw = lvalid || (!XD && (dead || keepq || keepf) && a0 + ll < line_end_i(a.n0));
@@ -534,7 +534,8 @@ __device__ __forceinline__ void sweep_tile(const A& args, const A& args_w, int t
         double x[L];
         double* ln = tile + l * a.rs_in + TG;
         const double keep0 = ln[HM], keepd = ln[HM + dim];
-        solve_line<L, OP>(ln, tab, a.fc, x);
+        const bool keepl = keepf && l >= nvalid;  // a line stored back as staged
+        solve_line<L, OP>(ln, tab, a.fc, x, keepl);
         if constexpr (PASS == PASS_GRAD) {
             // gradcal's metric factor dxi(d,d) (src/comsolver.F90:304-318)
             // on the lane's rows, loaded with the staging
@@ -548,7 +549,7 @@ __device__ __forceinline__ void sweep_tile(const A& args, const A& args_w, int t
         // which the half-wavefront has finished reading and nothing reads
         // again
         const int sub = lane & 31;
-        if (!keepf || l < nvalid) {
+        if (!keepl) {
 #pragma unroll
             for (int t = 0; t < L; ++t) ln[HM + tab.first + sub * L + t] = x[t];
         }

@@ -228,9 +228,13 @@ __device__ __forceinline__ void thomas_rows(const LineTab& tb, double (&x)[L]);
 // Solve the line held in LDS at ln (nodes -HM..dim+HM).  Called by a whole
 // wavefront; lanes 0-31 and 32-63 each solve their own line (same system),
 // lane sub of a half holds rows sub*L .. sub*L+L-1 in x[] on return.
+// keep: the half's line stays in LDS as it is (a line that the caller stores
+// back as staged; what x then holds is no solution).  Else the slots of its
+// rows may be written, which the caller overwrites with the solution.
 template <int L, int OP>
-__device__ __forceinline__ void solve_line(const double* ln, const LineTab& tb,
-                                           const FiltCoef* __restrict__ fc, double (&x)[L])
+__device__ __forceinline__ void solve_line(double* ln, const LineTab& tb,
+                                           const FiltCoef* __restrict__ fc, double (&x)[L],
+                                           bool keep = false)
 {
     constexpr int HW = OP == OP_DERIV ? 2 : 5;  // interior stencil half-width
     constexpr int W = L + 2 * HW;
@@ -294,9 +298,9 @@ __device__ __forceinline__ void solve_line(const double* ln, const LineTab& tb,
         // solution overwrites, and the owners take them from there.
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
         __builtin_amdgcn_wave_barrier();
-        double* row = const_cast<double*>(ln) + HM + tb.first;
-        if (sub < tb.nlo) row[sub] = cv;
-        if (31 - sub < tb.nhi) row[R - 1 - (31 - sub)] = cv;
+        double* row = ln + HM + tb.first;
+        if (sub < tb.nlo && !keep) row[sub] = cv;
+        if (31 - sub < tb.nhi && !keep) row[R - 1 - (31 - sub)] = cv;
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
         __builtin_amdgcn_wave_barrier();
 #pragma unroll
