@@ -11,7 +11,8 @@ import sys
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 SOURCES = [os.path.join(HERE, "csrc", "astr_solver.hip")]
-HEADERS = [os.path.join(HERE, "csrc", "line_engine.hpp"), os.path.join(ROOT, "include", "astr_hip.h")]
+HEADERS = [os.path.join(HERE, "csrc", h) for h in ("geo.hpp", "line_engine.hpp", "upwind.hpp")] + [
+    os.path.join(ROOT, "include", "astr_hip.h")]
 TARGET = os.path.join(HERE, "libastr_hip.so")
 
 FLAGS = [

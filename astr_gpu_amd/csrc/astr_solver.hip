@@ -73,21 +73,8 @@ constexpr int TXX = 8;     // lines per x tile: one per half-wavefront
 constexpr int TX = TXY;    // largest tile
 constexpr int WGT = 256;   // threads per sweep workgroup
 constexpr int TG = 3;      // LDS guard slots before each staged line
-constexpr int OI = 16;     // element offset of node i=0 in a row
-static_assert(OI % 16 == 0, "node i = 0 starts a 128-byte line");
 constexpr int LMAX = 16;   // rows per lane supported (line length <= 32*LMAX)
 constexpr int STATS_SLOTS = 1024;  // steps whose statistics stay on the device
-
-struct Geo {
-    int n[3];    // cells per axis (nodes 0..n)
-    long s[3];   // element stride per axis (s[0] = 1)
-    long org;    // element offset of node (0,0,0)
-};
-
-__host__ __device__ __forceinline__ long gidx(const Geo& g, int i, int j, int k)
-{
-    return g.org + i + j * g.s[1] + k * g.s[2];
-}
 
 // Node i = 0 of every row starts a 128-byte line (OI = 16 doubles, rows a
 // multiple of 16).  A kernel that writes nodes 0..n of a row also writes,
@@ -228,8 +215,10 @@ __device__ __forceinline__ void block_tile(int bid, int nq, int ntiles, int& til
     (void)ntiles;
 }
 
-// load / store through a 32-bit byte offset from a wave-uniform base (every
-// field is below 4 GB), so the address is one VGPR added to an SGPR pair
+// load / store through a 32-bit byte offset from a wave-uniform base, so the
+// address is one VGPR added to an SGPR pair: from the field's start where the
+// line sweeps run (axes of at most 505 cells: every field is below 4 GB), from
+// a plane's elsewhere
 // (every field is global memory: the accesses say so, so that pointers read
 // from an argument table rather than the kernel arguments also give global
 // rather than flat instructions).  Both are streaming (nontemporal): a
@@ -2739,7 +2728,8 @@ unsigned sensor_layout(SensorArgs& a)
     return (unsigned)((nb + 7) / 8 * 8);
 }
 
-// two doubles through a 32-bit byte offset, as ldc
+// two doubles through a 32-bit byte offset, as ldc (a plane's: an upwind
+// context's fields may be larger)
 typedef double d2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ d2 ldc2(const double* base, unsigned int boff)
 {
@@ -2796,9 +2786,10 @@ __global__ __launch_bounds__(256, 4) void k_ssf(SensorArgs a)
     if (!sensor_pair(a, c[0], c[1], c[2])) return;
     const int i = c[0], n0 = a.g.n[0];
     const bool two = i < n0;  // node i + 1 exists
-    const unsigned gi = (unsigned)gidx(a.g, i, c[1], c[2]), gb = gi * 8u;
+    const unsigned gb = plane_byte(a.g, i, c[1]);
+    const long pl0 = plane_elem(a.g, c[2]);
     double dv[2][9];
-    const double* P = a.prs;
+    const double* P = a.prs + pl0;
     const long s1 = a.g.s[1], s2 = a.p2d ? 0 : a.g.s[2];
     if constexpr (GRAD) {
         // (past a bounded end the loads meet the halo cells, which exist on
@@ -2811,7 +2802,7 @@ __global__ __launch_bounds__(256, 4) void k_ssf(SensorArgs a)
         }
 #pragma unroll
         for (int m = 0; m < 3; ++m) {
-            const double* f = a.vel[m];
+            const double* f = a.vel[m] + pl0;
             const d2 A = ldc2(f - 4, gb), B = ldc2(f - 2, gb), C = ldc2(f, gb);
             const d2 D = ldc2(f + 2, gb), E = ldc2(f + 4, gb);
             const double w0[7] = {A.y, B.x, B.y, C.x, C.y, D.x, D.y};
@@ -2837,7 +2828,7 @@ __global__ __launch_bounds__(256, 4) void k_ssf(SensorArgs a)
     } else {
 #pragma unroll
         for (int m = 0; m < 9; ++m) {
-            const d2 v = ldc2(a.dvel[m], gb);
+            const d2 v = ldc2(a.dvel[m] + pl0, gb);
             dv[0][m] = v.x;
             dv[1][m] = v.y;
         }
@@ -2866,8 +2857,9 @@ __global__ __launch_bounds__(256, 4) void k_ssf(SensorArgs a)
         const double dpdk = fabs(pk1[e] - 2.0 * p0 + pk0[e]) / (pk1[e] + 2.0 * p0 + pk0[e]);
         out[e] = div2 / (div2 + vort + 1.e-30) * uwd::max2(uwd::max2(dpdi, dpdj), dpdk);
     }
-    if (two) *(d2*)(a.ssf + gi) = d2{out[0], out[1]};
-    else a.ssf[gi] = out[0];
+    double* o = a.ssf + gidx(a.g, i, c[1], c[2]);
+    if (two) *(d2*)o = d2{out[0], out[1]};
+    else *o = out[0];
 }
 
 // ducrossensor, part 2 (src/commcal.F90:278-316): lshock = max of ssf over
@@ -2882,8 +2874,9 @@ __global__ __launch_bounds__(256) void k_ducros_flag(SensorArgs a)
     if (!sensor_pair(a, c[0], c[1], c[2])) return;
     const int i = c[0], n0 = a.g.n[0];
     const bool two = i < n0;
-    const unsigned gi = (unsigned)gidx(a.g, i, c[1], c[2]), gb = gi * 8u;
-    const double* f = a.ssf;
+    const long gi = gidx(a.g, i, c[1], c[2]);
+    const unsigned gb = plane_byte(a.g, i, c[1]);
+    const double* f = a.ssf + plane_elem(a.g, c[2]);
     double m[2] = {0.0, 0.0};
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
@@ -2928,8 +2921,8 @@ __global__ __launch_bounds__(256) void k_ducros_flag(SensorArgs a)
                 if (nt == 3) t = t < 0 ? t + n : (t > n ? t - n : t);
                 const int w = min(max(t, 0), n);
                 const bool zero = (t < 0 && !lo_end(nt)) || (t > n && !hi_end(nt));
-                if (d == 0) v[o].x = f[gi + w - i];
-                else v[o] = *(const d2*)(f + gi + (w - t0) * st);
+                if (d == 0) v[o].x = a.ssf[gi + w - i];
+                else v[o] = *(const d2*)(a.ssf + gi + (w - t0) * st);
                 if (zero) v[o] = d2{0.0, 0.0};
             }
 #pragma unroll
@@ -6312,15 +6305,8 @@ int astr_create(const astr_params* p, int32_t device, astr_ctx** out)
     if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess)
         return cleanup(fail(ASTR_E_HIP, "hipStreamCreate failed"));
 
-    for (int d = 0; d < 3; ++d) c->g.n[d] = dims[d];
-    c->pi = ((OI + dims[0] + 1 + HM) + 15) / 16 * 16;
-    c->pj = dims[1] + 1 + 2 * HM;
-    c->pk = dims[2] + 1 + 2 * HM;
+    c->g = padded_geo(dims, c->pi, c->pj, c->pk);
     c->nfield = c->pi * c->pj * c->pk;
-    c->g.s[0] = 1;
-    c->g.s[1] = c->pi;
-    c->g.s[2] = c->pi * c->pj;
-    c->g.org = OI + HM * c->g.s[1] + HM * c->g.s[2];
     const int nfields = 5 + 6 + 5 + 5 + 9 + 3 + 15 + 1 + 2 + (p->convection != 0 ? 1 : 0) +
                         (p->convection == 2 ? 20 : 0);
     if (hipMalloc(&c->base, sizeof(double) * c->nfield * nfields) != hipSuccess)

@@ -27,9 +27,10 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include "geo.hpp"
+
 namespace astr {
 
-constexpr int HM = 5;    // halo width, src/commvar.F90:190
 constexpr int LPL = 32;  // lanes per line
 
 enum LineOp : int { OP_DERIV = 0, OP_FILTER = 1 };
