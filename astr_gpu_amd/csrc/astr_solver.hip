@@ -6536,7 +6536,8 @@ int astr_upload_geom(astr_ctx* c, const double* jacob, const double* dxi)
             double* base = nullptr;
             if (hipMalloc(&base, sizeof(double) * c->nfield * 9) != hipSuccess)
                 return fail(ASTR_E_NOMEM, "device allocation of the metric fields failed");
-            HIPCHK(hipMemset(base, 0, sizeof(double) * c->nfield * 9));
+            // (not cleared: the uploads write every element, and a clear on
+            // the null stream would not be ordered before them)
             for (int m = 0; m < 9; ++m) c->dxf[m] = base + (long)m * c->nfield;
         }
         for (int d = 0; d < 3; ++d)
