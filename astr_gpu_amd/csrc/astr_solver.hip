@@ -1857,7 +1857,10 @@ __global__ __launch_bounds__(64, L <= 6 ? 4 : 3) void k_row_flux(RowArgs ra)
     const unsigned dhj = (unsigned)((hj - j) * (int)a.g.s[1]) * 8u;
     const unsigned dhk = (unsigned)((hk - k) * (int)a.g.s[2]) * 8u;
     const double xy = a.xi[1][j + HM], xz = a.xi[2][k + HM];
-    double st[3] = {0.0, 0.0, 0.0};
+    // the row's sums of the statistics, double-double from node to node: a
+    // row has up to 8 nodes to a lane, and k_stats keeps plain additions to
+    // the 64 lanes of one wavefront too
+    double st[3] = {0.0, 0.0, 0.0}, sl[3] = {0.0, 0.0, 0.0};
 #pragma unroll 1
     for (int c0 = 0; c0 < lend; c0 += 64) {
         const int c = c0 + lane;
@@ -1889,7 +1892,11 @@ __global__ __launch_bounds__(64, L <= 6 ? 4 : 3) void k_row_flux(RowArgs ra)
                 double t[3];
                 stats_of(vc, rho, nd.u, T, dv, t[0], t[1], t[2]);
 #pragma unroll
-                for (int m = 0; m < 3; ++m) st[m] += t[m];
+                for (int m = 0; m < 3; ++m) {
+                    double e;
+                    two_sum(st[m], t[m], st[m], e);
+                    sl[m] += e;
+                }
             }
             if (ra.keep_grad) {
 #pragma unroll
@@ -1979,11 +1986,12 @@ __global__ __launch_bounds__(64, L <= 6 ? 4 : 3) void k_row_flux(RowArgs ra)
 #pragma unroll
         for (int off = 32; off > 0; off >>= 1)
 #pragma unroll
-            for (int m = 0; m < 3; ++m) st[m] += __shfl_xor(st[m], off, 64);
+            for (int m = 0; m < 3; ++m)
+                dd_add(st[m], sl[m], __shfl_xor(st[m], off, 64), __shfl_xor(sl[m], off, 64));
         if (lane == 0)
             for (int m = 0; m < 3; ++m) {
                 a.part[6 * (long)blockIdx.x + 2 * m] = st[m];
-                a.part[6 * (long)blockIdx.x + 2 * m + 1] = 0.0;
+                a.part[6 * (long)blockIdx.x + 2 * m + 1] = sl[m];
             }
     }
 }
