@@ -1786,9 +1786,15 @@ __device__ __forceinline__ void row_back(const LineTab& tab, int sub, double* ln
 // stay on the chip).  Per stage, three kernels -> one: 256^3 1689 -> 1060 us
 // (4.25 TB/s), 128^3 259 -> 152 us, 64^3 56 -> 33 us.  Registers: up to L = 6
 // the table of the line system is held over the solves within 128 of them (4
-// waves per SIMD); above, the five LDS rows allow 3 waves.
+// waves per SIMD); up to L = 10 within 168 (3 waves); above, the five LDS rows
+// let 11 wavefronts and fewer on a CU, so 2 waves' 256 registers cost nothing.
+// (A 256^3 stage's rows are L = 9.  With 168 registers the rows of L >= 11
+// spilled, up to 227 of them: a step of 345x64x64 took 1466 us against 1437,
+// 409 1838 against 1642, 473 2319 against 1962, 505 2721 against 2346, and the
+// separate kernels 1580, 1803, 2092 and 2426.  At L = 10, 313 cells, 3 waves
+// measured 1277 and 2 waves 1301.)
 template <int L, bool STATS>
-__global__ __launch_bounds__(64, L <= 6 ? 4 : 3) void k_row_flux(RowArgs ra)
+__global__ __launch_bounds__(64, L <= 6 ? 4 : L <= 10 ? 3 : 2) void k_row_flux(RowArgs ra)
 {
     extern __shared__ double buf[];
     const PtArgs& a = ra.p;
