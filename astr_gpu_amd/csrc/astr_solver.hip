@@ -5234,13 +5234,22 @@ int do_stats(astr_ctx* c, double* out)
 // needs them only while it runs: at most PIN_MAX of them, lent to one worker
 // of one call at a time, freed when the last context goes.
 
-constexpr size_t PIN_HALF = (size_t)2 << 20;  // bytes of a half: a worker fills one while
-                                              // the other's DMA runs
+// Bytes of a half (a worker fills one while the other's DMA runs).  The
+// runtime hands out pinned memory again at once (14 us) while less than 4 MB
+// of it are asked for; 4 MB take 300 us, the next device allocation 300 and
+// the first touch 800-1600.  So where the chunks fit (two workers, boxes up to
+// about 40^3) the buffers start small, and grow for a larger transfer.  (A
+// context made, filled, read and closed with no other alive, in ms before
+// there were pinned buffers / with 4 MB ones from the start / so: 16^3 1.41 /
+// 2.1-2.3 / 1.35-1.5, 40x32x36 3.3 / 4.4-4.7 / 2.7-3.9.  Halves of 1 MB
+// throughout took 1.3 times as long at 256^3.)
+constexpr size_t PIN_SMALL = ((size_t)1 << 20) - 8192, PIN_HALF = (size_t)2 << 20;
 constexpr int PIN_MAX = 16;                   // buffers of two halves: 64 MB in all
 constexpr int XFER_THREADS = 8;               // workers of one call
 
 struct PinBuf {
     double* p = nullptr;
+    size_t half = 0;  // bytes of each half
     int device = -1;  // of the events
     hipEvent_t ev[2] = {nullptr, nullptr};  // the DMA of each half
     ~PinBuf()
@@ -5264,23 +5273,44 @@ PinPool& pin_pool()
     return *p;
 }
 
+// b with halves of at least `half` bytes; false where pinned memory is refused
+bool pin_fit(PinBuf* b, size_t half)
+{
+    if (b->half >= half) return true;
+    if (b->p) (void)hipHostFree(b->p);
+    b->p = nullptr;
+    b->half = 0;
+    if (hipHostMalloc(&b->p, 2 * half, hipHostMallocPortable) != hipSuccess) {
+        (void)hipGetLastError();
+        b->p = nullptr;
+        return false;
+    }
+    b->half = half;
+    return true;
+}
+
 // up to `want` buffers, at least one: waits while every buffer is lent
 // (their holders wait for nobody).  Empty where pinned memory is refused.
-std::vector<PinBuf*> pin_take(int want)
+std::vector<PinBuf*> pin_take(int want, size_t half)
 {
     PinPool& P = pin_pool();
     std::vector<PinBuf*> got;
     std::unique_lock<std::mutex> lk(P.mu);
     P.cv.wait(lk, [&] { return !P.idle.empty() || P.made < PIN_MAX; });
     while ((int)got.size() < want && !P.idle.empty()) {
-        got.push_back(P.idle.back());
+        PinBuf* b = P.idle.back();
         P.idle.pop_back();
+        if (pin_fit(b, half)) {
+            got.push_back(b);
+            continue;
+        }
+        delete b;
+        --P.made;
+        P.cv.notify_all();  // one may be made in its place
     }
     while ((int)got.size() < want && P.made < PIN_MAX) {
         PinBuf* b = new PinBuf();
-        if (hipHostMalloc(&b->p, 2 * PIN_HALF, hipHostMallocPortable) != hipSuccess) {
-            (void)hipGetLastError();
-            b->p = nullptr;
+        if (!pin_fit(b, half)) {
             delete b;
             break;
         }
@@ -5360,7 +5390,11 @@ int transfer(astr_ctx* c, const std::vector<HostField>& fields, bool up)
     // 2 MB).  (Downloads of a 41x33x37 box, 11 MB: 2 workers 0.41 ms, 6 0.73;
     // of a 97x65x81 field, 7 MB up and down: 1 worker 0.51 ms, 4 0.79.)
     const int want = (int)std::min<double>(XFER_THREADS, std::max(1.0, std::sqrt(bytes / 2e6)));
-    std::vector<PinBuf*> bufs = pin_take(want);
+    // chunks of at most a half, and a few for each worker's two halves
+    const long chunk = std::max<long>(
+        std::min<long>((long)(PIN_HALF / sizeof(double)), (total / want + 3) / 4), 1 << 16);
+    const size_t need = sizeof(double) * (size_t)std::min(chunk, c->nfield);
+    std::vector<PinBuf*> bufs = pin_take(want, need <= PIN_SMALL ? PIN_SMALL : PIN_HALF);
     // where pinned memory is refused, one worker through plain memory
     PinBuf plain;
     std::unique_ptr<double[]> mem;
@@ -5368,16 +5402,19 @@ int transfer(astr_ctx* c, const std::vector<HostField>& fields, bool up)
         mem.reset(new (std::nothrow) double[2 * PIN_HALF / sizeof(double)]);
         if (!mem) return fail(ASTR_E_NOMEM, "host buffer");
         plain.p = mem.get();
+        plain.half = PIN_HALF;
     }
     const int nw = std::max(1, (int)bufs.size());
-    // chunks of at most a half, and a few for each worker's two halves
-    const long chunk = std::max<long>(
-        std::min<long>((long)(PIN_HALF / sizeof(double)), (total / nw + 3) / 4), 1 << 16);
     const long per = (c->nfield + chunk - 1) / chunk, nchunks = per * (long)fields.size();
+    // one worker that fills neither half twice (one field of up to 1 MB, a
+    // box of about 32^3): it waits for the stream, which returns 7 us sooner
+    // than an event (a line operator on a 16^3 box 75 -> 60 us, as long as
+    // plain copies took; 28^3 126 -> 113)
+    const bool lone = nw == 1 && nchunks <= 2;
     std::atomic<long> next{0};
     std::atomic<int> err{(int)hipSuccess};
     auto work = [&](PinBuf* b) {
-        double* half[2] = {b->p, b->p + PIN_HALF / sizeof(double)};
+        double* half[2] = {b->p, b->p + b->half / sizeof(double)};
         hipEvent_t* const ev = b->ev;
         long at[2] = {-1, -1};  // the chunk whose DMA is in a half
         auto ok = [&](hipError_t e) {
@@ -5388,7 +5425,7 @@ int transfer(astr_ctx* c, const std::vector<HostField>& fields, bool up)
             if (at[h] < 0) return;
             const long k = at[h];
             at[h] = -1;
-            if (!ok(hipEventSynchronize(ev[h])) || up) return;
+            if (!ok(lone ? hipStreamSynchronize(c->stream) : hipEventSynchronize(ev[h])) || up) return;
             const long e0 = (k % per) * chunk;
             copy_chunk(c, fields[k / per], half[h], e0, std::min(e0 + chunk, c->nfield), false);
         };
@@ -5417,7 +5454,7 @@ int transfer(astr_ctx* c, const std::vector<HostField>& fields, bool up)
                     break;
                 }
                 at[h] = k;
-                if (!ok(hipEventRecord(ev[h], c->stream))) {
+                if (!lone && !ok(hipEventRecord(ev[h], c->stream))) {
                     (void)hipStreamSynchronize(c->stream);
                     at[h] = -1;
                     break;
