@@ -1752,6 +1752,8 @@ struct RowArgs {
 // doubles per x halo node of k_row_flux's side rows: the image's sigma (3) and
 // heat flux, the node's q (5), p, u and J
 constexpr int ROW_STRIP = 12;
+// rows per lane up to which the statistics' low words sit in LDS
+constexpr int ROW_LO_LDS = 3;
 
 __device__ __forceinline__ void wave_sync()
 {
@@ -1863,10 +1865,17 @@ __global__ __launch_bounds__(64, L <= 6 ? 4 : L <= 10 ? 3 : 2) void k_row_flux(R
     const unsigned dhj = (unsigned)((hj - j) * (int)a.g.s[1]) * 8u;
     const unsigned dhk = (unsigned)((hk - k) * (int)a.g.s[2]) * 8u;
     const double xy = a.xi[1][j + HM], xz = a.xi[2][k + HM];
-    // the row's sums of the statistics, double-double from node to node: a
-    // row has up to 8 nodes to a lane, and k_stats keeps plain additions to
-    // the 64 lanes of one wavefront too
+    // the row's sums of the statistics, double-double over a lane's nodes (up
+    // to 8); plain additions, as in stats_block_sum, only over the 64 lanes
+    // (The low words of short rows sit in LDS: with them in registers the
+    // instance takes 101, 4 waves per SIMD instead of 5, and the 4225 rows of
+    // a 64^3 box are 129 more than the chip then holds at once.  Stage 1 with
+    // the statistics, plain sums -> these: 64^3 34.7 -> 36.4 us, 112x81x64
+    // 54.7 -> 56.1.)
     double st[3] = {0.0, 0.0, 0.0}, sl[3] = {0.0, 0.0, 0.0};
+    double* const slo = side + ROW_STRIP * 2 * HM + lane;
+    if (STATS && L <= ROW_LO_LDS)
+        for (int m = 0; m < 3; ++m) slo[64 * m] = 0.0;
 #pragma unroll 1
     for (int c0 = 0; c0 < lend; c0 += 64) {
         const int c = c0 + lane;
@@ -1901,7 +1910,8 @@ __global__ __launch_bounds__(64, L <= 6 ? 4 : L <= 10 ? 3 : 2) void k_row_flux(R
                 for (int m = 0; m < 3; ++m) {
                     double e;
                     two_sum(st[m], t[m], st[m], e);
-                    sl[m] += e;
+                    if (L <= ROW_LO_LDS) slo[64 * m] += e;
+                    else sl[m] += e;
                 }
             }
             if (ra.keep_grad) {
@@ -1989,11 +1999,15 @@ __global__ __launch_bounds__(64, L <= 6 ? 4 : L <= 10 ? 3 : 2) void k_row_flux(R
             stb(ra.qrhs[m], g0 + (unsigned)(c * 8), buf[m * rs + TG + HM + min(c, n)]);
     }
     if (STATS) {
+        if (L <= ROW_LO_LDS)
+            for (int m = 0; m < 3; ++m) sl[m] = slo[64 * m];
 #pragma unroll
         for (int off = 32; off > 0; off >>= 1)
 #pragma unroll
-            for (int m = 0; m < 3; ++m)
-                dd_add(st[m], sl[m], __shfl_xor(st[m], off, 64), __shfl_xor(sl[m], off, 64));
+            for (int m = 0; m < 3; ++m) {
+                st[m] += __shfl_xor(st[m], off, 64);
+                sl[m] += __shfl_xor(sl[m], off, 64);
+            }
         if (lane == 0)
             for (int m = 0; m < 3; ++m) {
                 a.part[6 * (long)blockIdx.x + 2 * m] = st[m];
@@ -4588,7 +4602,8 @@ template <bool STATS>
 int launch_row_flux(astr_ctx* c, const RowArgs& r)
 {
     const dim3 grid((unsigned)((c->g.n[1] + 1) * (c->g.n[2] + 1)));
-    const size_t lds = sizeof(double) * (5 * (size_t)r.rs + ROW_STRIP * 2 * HM);
+    const size_t lds = sizeof(double) * (5 * (size_t)r.rs + ROW_STRIP * 2 * HM +
+                                         (STATS && c->L[0] <= ROW_LO_LDS ? 3 * 64 : 0));
     switch (c->L[0]) {
 #define CASE(LL)                                                                          \
     case LL:                                                                              \
