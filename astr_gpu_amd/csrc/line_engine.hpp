@@ -57,9 +57,10 @@ constexpr int CLW = 11, CLS = 12;  // width of a closure row, its stride in cl
 constexpr int CLR = 5;             // most closure rows at an end
 // Rows per lane up to which the filter's closure rows are taken one per lane
 // (below).  Per launch: 64^3 (L = 3) y/z 17.7 -> 15.4 us and x 13.8 -> 12.4,
-// 112x81x64 y/z 30.4 -> 25.8, 40x32x36 (L = 2) 9.9 -> 7.1; at L = 5
-// (128^3) 56 -> 63 and at L = 9 (256^3) 320 -> 372: there the rows after each
-// other hide behind the other wavefronts' loads, and the table's do not.
+// 112x81x64 y/z 30.4 -> 25.8, 40x32x36 (L = 2) 9.9 -> 7.1; at L = 4 (96^3)
+// y/z 32.6 -> 33.6 and (112^3) 43.4 -> 45.6, at L = 5 (128^3) 56 -> 63 and at
+// L = 9 (256^3) 320 -> 372: there the rows after each other hide behind the
+// other wavefronts' loads, and the table's do not.
 constexpr int CL_LANES_MAX = 3;
 
 // filter_coefficient_cal tables (src/filter.F90:299-432) used on the path.

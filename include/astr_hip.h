@@ -257,11 +257,12 @@ int astr_adjoint_enstrophy(astr_ctx *ctx, int32_t nsteps, double dt, int32_t ckp
 /* Kernel time since timing was (re)enabled with astr_set_timing(ctx, 1),
  * in milliseconds, per kernel family (HIP events on the solver's stream):
  * [0] filter sweeps, [1] boucon and qswap, [2] gradient (central on a
- * rectilinear viscous box: y and z), [3] central: sigma/qflux and the flux
- * of each axis, there with the x gradient and x flux derivative, which the
- * same kernel forms; upwind steps: the shock sensor, [4] statistics, [5]
- * flux sweeps (central: inviscid and viscous flux derivatives, the z sweep
- * applying the RK3 combine; upwind: interface fluxes), [6] update (central: primitives; upwind: RK3 combine and
+ * rectilinear viscous box with the compact gradient: y and z), [3] central:
+ * sigma/qflux and the flux of each axis, there with the x gradient and x
+ * flux derivative, which the same kernel forms; upwind steps: the shock
+ * sensor, [4] statistics, [5] flux sweeps (central: inviscid and viscous
+ * flux derivatives, the z sweep applying the RK3 combine; upwind: interface
+ * fluxes), [6] update (central: primitives; upwind: RK3 combine and
  * primitives), [7] total, [8] shock sensor of astr_rhscal.
  * astr_rk3_step(s) fill 0-7; astr_rhscal of an upwind context fills 2, 5,
  * 7 and 8.  astr_rk3_steps restarts the count at each call.  Mode 1 puts
